@@ -138,7 +138,7 @@ struct AttnArgs {
   float* part;             // decode: o [kDecMaxChunks][kAttnMaxQ][256] then (m, l) [kDecMaxChunks][kAttnMaxQ][2];
                            // batched prefill: (m, l, o[256]) [row][kPrefillChunks][n_q]
   float* attn_out;         // decode [n_q * 256]
-  uint16_t* pf_out;        // batched prefill: hi plane [row][n_q * 256], then lo plane
+  uint16_t* pf_out;        // batched prefill: the O GEMM's input, [row][n_q * 8][2][32]
   float* q_dbg;            // decode, optional: normed+roped q of this token
   // batched prefill: prompt row r sits at position pf_start + r; q of every
   // row is already normed + roped in `qkv`, K/V of every position are in the
@@ -148,20 +148,21 @@ struct AttnArgs {
   int pf_chunk;
 };
 
-// Prefill GEMM on bf16 MFMA: C[M x N] = A[M x K] * W[N x K]^T. A comes as two
-// bf16 planes (hi = bf16(x), lo = bf16(x - hi)); W as its int8 values in
-// bf16 (exact) with the fp32 scale of every 32-wide block, applied to each
-// block's MFMA partial in fp32.
+// Prefill GEMM on bf16 MFMA: C[M x N] = A[M x K] * W[N x K]^T. A comes as
+// bf16 hi / lo (hi = bf16(x), lo = bf16(x - hi)), a row's 32-blocks one after
+// the other, each 32 hi then 32 lo values; W as its int8 values in bf16
+// (exact) in MFMA operand order with the fp32 scale of every 32-wide block,
+// applied to each block's MFMA partial in fp32 (launch_q8_bf16 writes both).
 struct GemmArgs {
-  const uint16_t* A;       // hi plane [M][K], then lo plane [M][K]
-  const uint16_t* W;       // [N][K]
-  const float* D;          // [N][K / 32]
+  const uint16_t* A;       // [M][K / 32][2][32]
+  const uint16_t* W;       // [N / 16][K / 32][64][8]
+  const float* D;          // [N / 16][K / 32][16]
   int M, N, K;
   int ks;                  // K slices (1..kGemmMaxSlices, EPI_OUT only): slice z covers K/ks and writes C + z M N
-  int bn;                  // block tile width: 128, or 144 / 96 (EPI_OUT: 4 waves of 32 x 144 / 64 x 48)
+  int tile;                // GemmTileId
   float* C;                // EPI_OUT: [M][N] per slice
-  uint16_t* act;           // EPI_GEGLU: hi plane [M][N/2], then lo plane; gate / up rows
-                           // alternate in groups of 16 (16 gate rows, then their up rows)
+  uint16_t* act;           // EPI_GEGLU: [M][N / 64][2][32], the 32 inputs of a block in act_slot order;
+                           // gate / up rows alternate in groups of 16 (16 gate rows, then their up rows)
 };
 
 // Row-wise prefill helpers: one block per prompt row.
@@ -180,7 +181,7 @@ struct RowArgs {
   const float* w_post;
   const float* w_pre;
   float* res_out;          // [M][H] new residual stream
-  uint16_t* x_out;         // normed GEMM input: hi plane [M][H], then lo plane
+  uint16_t* x_out;         // normed GEMM input, [M][H / 32][2][32]
   float* last_hidden;      // optional: row M-1 of res_out (per-layer history)
   // KV: k/v of each row into the cache, q heads normed + roped in place
   const float* qkv;
@@ -337,17 +338,35 @@ int launch_repack_gum(const uint8_t* src, uint8_t* dst, long long rows, int K, i
 // Class-major copy of the CI = 1 LM head (rows a multiple of 16384).
 int launch_class_major(const uint8_t* src, uint8_t* dst, long long rows, int Kp, void* stream);
 // GGUF Q8_0 rows -> prefill GEMM weights: source row r to row r + off, or
-// with half = 16 to (r / 16) * 32 + r % 16 + off (gate: off 0, up: off 16).
+// with half = 16 to (r / 16) * 32 + r % 16 + off (gate: off 0, up: off 16);
+// act_order: inputs permuted to the GeGLU epilogue's order (down).
 int launch_q8_bf16(const uint8_t* src, uint16_t* wb, float* wd, long long rows, int K, long long off, int half,
-                   void* stream);
+                   int act_order, void* stream);
 int launch_seen_add(uint32_t* seen, DevState* st, const int32_t* ids, int n, int V, void* stream);
 int launch_prefill_attention(const AttnArgs& a, int M, void* stream);
 int launch_gemm(int epi, const GemmArgs& a, void* stream);
 int launch_rows_embed(const RowArgs& a, void* stream);
 int launch_rows_resid(const RowArgs& a, void* stream);
 int launch_rows_kv(const RowArgs& a, void* stream);
-constexpr int kGemmMaxSlices = 4;   // K slices of a prefill GEMM (summed by the consumer)
-constexpr int kQkvMaxSlices = 2;    // ... of the QKV GEMM (summed by k_rows_kv)
+// Block tiles of the prefill GEMM (rows x features).
+enum GemmTileId { GT_32x64, GT_32x128, GT_32x192, GT_64x128, GT_64x192, GT_64x256, GT_128x256, GT_COUNT };
+struct GemmTile {
+  int mi, nj;       // 16 mi rows, 64 nj features
+  bool out, geglu;  // epilogues it is built for
+  float lat, thr;   // us per 32-wide step: alone on a CU / added by each further block of the CU
+};
+// lat and thr: least-squares fit of 2000 timings, 16 to 4096 rows x the GEMM
+// shapes of Gemma-3 270M and 1B x 1 to 8 K slices, weights from HBM (12% rms).
+constexpr GemmTile kGemmTiles[GT_COUNT] = {
+    {2, 1, true, false, .182f, .116f}, {2, 2, true, true, .252f, .201f},  {2, 3, true, false, .329f, .297f},
+    {4, 2, true, true, .361f, .355f},  {4, 3, true, false, .463f, .473f}, {4, 4, false, true, .605f, .485f},
+    {8, 4, false, true, .955f, .919f}};
+constexpr int kGemmMaxSlices = 8;   // K slices of a prefill GEMM (summed by the consumer)
+// Slices that the output buffers of an M-row GEMM hold: few rows need more
+// blocks and their slices are small.
+constexpr int kGemmFewRows = 512;
+inline int gemm_slices(int M) { return M <= kGemmFewRows ? kGemmMaxSlices : 4; }   // O, down
+inline int qkv_slices(int M) { return M <= kGemmFewRows ? 4 : 2; }
 constexpr int kPrefillChunks = 16;   // key chunks per query tile in the batched prefill attention
 constexpr int kPrefillMinChunk = 160;
 // Longest key span of a 32-row query tile of a prefill of M rows at `start`.

@@ -20,8 +20,7 @@
 // A batched prefill runs per layer the bf16-MFMA GEMMs (k_gemm: int8 weights
 // exact in bf16, activations split into bf16 hi + lo), the row kernels
 // (norms, residuals, QK-norm + RoPE + KV store) and the MFMA attention
-// k_attn_pf (+ k_attn_pf_merge for long spans); the GEMM tiles are 128 x 128,
-// or 128 x 144 for 1152-wide outputs with a K split.
+// k_attn_pf (+ k_attn_pf_merge for long spans).
 //
 // On this multi-XCD part a device-scope fence is a whole-L2 write-back, so
 // kernels never fence and never exchange data across blocks of one launch:
@@ -909,6 +908,7 @@ typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ int a_slot(int e);   // below, with the GEMM's A rows
 // The same split for two values at once, as packed bf16 pairs (element 0 in
 // the low half): one packed conversion for hi, hi widened back by a shift and
 // a mask, one packed conversion for lo.
@@ -1170,11 +1170,13 @@ __global__ __launch_bounds__(512, 1) void k_attn_pf(AttnArgs a) {
     const int orow = qt * kPfRows + rt * 16 + 4 * g + r;
     if (orow >= M) continue;
     if (nkc == 1) {
-      uint16_t* out = a.pf_out + (size_t)orow * nq * kHeadDim + h * kHeadDim + c16;
-      const size_t plane = (size_t)M * nq * kHeadDim;
+      uint16_t* out = a.pf_out + ((size_t)orow * nq + h) * kHeadDim * 2;
       const float il = 1.f / lr[r];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) split_bf16(o[i][r] * il, &out[16 * i], &out[plane + 16 * i]);
+      for (int i = 0; i < 16; ++i) {
+        const int e = a_slot(16 * i + c16);
+        split_bf16(o[i][r] * il, &out[e], &out[e + 32]);
+      }
     } else {
       float* pp = a.part + (((size_t)orow * kPrefillChunks + kc) * nq + h) * (2 + kHeadDim);
 #pragma unroll
@@ -1237,12 +1239,11 @@ __global__ __launch_bounds__(256) void k_attn_pf_merge(AttnArgs a) {
       }
     }
   }
-  const size_t e = (size_t)row * nq * kHeadDim + h * kHeadDim + 4 * d4;
-  const size_t lo = (size_t)a.pf_rows * nq * kHeadDim;
-  split_bf16(O.x / L, &a.pf_out[e], &a.pf_out[lo + e]);
-  split_bf16(O.y / L, &a.pf_out[e + 1], &a.pf_out[lo + e + 1]);
-  split_bf16(O.z / L, &a.pf_out[e + 2], &a.pf_out[lo + e + 2]);
-  split_bf16(O.w / L, &a.pf_out[e + 3], &a.pf_out[lo + e + 3]);
+  uint16_t* out = a.pf_out + ((size_t)row * nq + h) * kHeadDim * 2 + a_slot(4 * d4);
+  bf16x4 hi, lo;
+  split4_bf16(O.x / L, O.y / L, O.z / L, O.w / L, hi, lo);
+  *(bf16x4*)out = hi;
+  *(bf16x4*)(out + 32) = lo;
 }
 
 // ---------------------------------------------------------------------------
@@ -1258,152 +1259,225 @@ __global__ __launch_bounds__(256) void k_attn_pf_merge(AttnArgs a) {
 // added to the output in fp32 -- the linearQ8 structure (shaders.ts:123-142)
 // with the block sum on the matrix cores.
 //
-// Block tile 128 (rows) x BN (features) x 64 (k step), four waves of
-// 16 NI x 16 NJ (NI x NJ MFMA tiles): 2 x 2 waves of 64 x 64 (BN = 128),
-// 4 x 1 waves of 32 x 144 (BN = 144; 1152-wide outputs then split into 8
-// tiles, so that a K split of 4 fills the 512 block slots of the chip
-// exactly) or 2 x 2 waves of 64 x 48 (BN = 96; the 1536 QKV outputs in 16
-// tiles, so that a K split of 2 gives 512 blocks at 2048 rows). LDS rows are padded to 72 bf16 so that the 16 lanes of a lane
-// group (16 rows, one 16-byte chunk) cover all banks; the next step's global
-// loads are issued before the current step's MFMAs.
+// A block is four waves side by side along the features: each owns 16 NJ
+// weight rows and all 16 MI activation rows of the block. Weights are laid
+// out as MFMA operands (one contiguous KB per 16 rows x 32 inputs), so they
+// go from L2 straight to the registers of the one wave that uses them, PW
+// steps ahead; only A, which the four waves share, passes through LDS (two
+// stages of one 32-wide step, one barrier per step, PA steps of global loads
+// in flight in registers). A 64 x 256 block so reads 16 bytes of LDS per
+// MFMA cycle and SIMD where a 2 x 2 wave layout with W in LDS too read 24 and
+// wrote 12, and its operand reads are prefetched one row tile ahead.
+// What bounds it: at thousands of rows the power limit (a 64 x 256 tile keeps
+// the matrix cores busy 71% of the cycles at the 1.64 GHz left under that
+// load, a 128 x 256 one 63% at 1.83 GHz, in the same time), at a hundred rows
+// the latency of a step. The larger tiles use each weight for more rows and
+// win where weights come from HBM, the small ones start more blocks. Gate/up
+// of the 1B shape (N 13824, K 1152), weights cold: 4096 rows 283 -> 230 us,
+// 2048 rows 155 -> 125 us, 187 rows 33 -> 27 us against a 128 x 128 tile with
+// both operands in LDS; gate/up of the 270M shape at 64 rows 20 -> 8.5 us.
+//
+// A rows are [K / 32][hi 32 | lo 32] bf16: one 128-byte line per 32-block.
+// In LDS a 16-row tile's (plane, 8-wide chunk g) is 256 bytes of 16 rows, row
+// r at slot r ^ (4 plane + g): the eight lanes that write one line and the
+// eight that read one chunk each cover all banks. Rows past M are outside
+// the buffer descriptors: their loads give zeros, their stores are dropped.
 // ---------------------------------------------------------------------------
-constexpr int kGBM = 128, kGBP = 72;
+__device__ __forceinline__ u32x4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (uint32_t)bytes, 0x00020000);
+}
 
-template <int EPI, int NI, int NJ>
-__global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs a) {
-  constexpr int WM = 128 / (16 * NI), WN = 4 / WM;   // waves along rows / features
-  constexpr int BN = WN * 16 * NJ;
-  constexpr int WI = (BN * 8 + 255) / 256;   // 16-byte W chunks per thread and step
-  constexpr int DI = (BN * 2 + 255) / 256;   // block scales per thread and step
-  static_assert(WM * WN == 4 && WM * 16 * NI == kGBM, "four waves cover the 128-row tile");
+// Position of input f of a 32-block in the planes that the GeGLU epilogue
+// writes: a lane holds inputs c and 16 + c, stored as one dword, so the
+// down weights carry their inputs in this order.
+__device__ __forceinline__ int act_slot(int f) { return 2 * (f & 15) + (f >> 4); }
+
+template <int EPI, int MI, int NJ, int PW, int PA, int OCC>
+__global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
   static_assert(EPI == EPI_OUT || NJ % 2 == 0, "GeGLU pairs adjacent column tiles");
-  __shared__ __align__(16) uint16_t Ah[kGBM * kGBP];
-  __shared__ __align__(16) uint16_t Al[kGBM * kGBP];
-  __shared__ __align__(16) uint16_t Ws[BN * kGBP];
-  __shared__ float Ds[BN * 2];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int g = lane >> 4, c16 = lane & 15;
-  const int M = a.M, K = a.K;
+  constexpr int BM = 16 * MI, BN = 64 * NJ;
+  constexpr int AC = (BM * 8 + 255) / 256;   // 16-byte A chunks per thread and step
+  constexpr int SL = PW + 1;                 // weight register stages
+  static_assert(BM * 8 % 256 == 0, "whole chunks");
+  __shared__ __align__(16) uint8_t As[2][BM * 128];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int M = a.M, N = a.N, KB = a.K / 32;
   // Tile order: workgroups go to the XCDs round-robin (from an XCD that
   // depends on earlier dispatches), so the blocks with one value of b % 8
   // (launch order) share an XCD; they take the contiguous range
   // [(b % 8) G / 8, (b % 8 + 1) G / 8) of an order with the K slice
-  // slowest, then groups of 4 tile rows with the rows fastest, so that the
-  // blocks sharing an XCD's L2 share A rows and W tiles (fewer L2 misses).
+  // slowest, then groups of 8 tile rows with the rows fastest, so that the
+  // blocks sharing an XCD's L2 share A rows and W tiles (fewer L2 misses;
+  // groups of 4, 8 or 16 are within 1%, of 2 4% slower).
+  constexpr int GROUP = 8;
   const int NT = gridDim.x, MT = gridDim.y, G = NT * MT * gridDim.z;
   const int bid = blockIdx.x + NT * (blockIdx.y + MT * blockIdx.z);
   const int L = (G % 8 == 0) ? (bid % 8) * (G / 8) + bid / 8 : bid;
   const int kz = L / (NT * MT), Lp = L % (NT * MT);
-  const int fm = (Lp / (4 * NT)) * 4, gm = min(MT - fm, 4);
-  const int m0 = (fm + (Lp % (4 * NT)) % gm) * kGBM, n0 = ((Lp % (4 * NT)) / gm) * BN;
-  const int kn = K / a.ks;   // this block's K slice [kz kn, (kz + 1) kn)
-  const int wm = (wv / WN) * 16 * NI, wn = (wv % WN) * 16 * NJ;
-  const size_t MK = (size_t)M * K;
-  // staging: rows tid / 8 + 32 i, 16-byte chunk tid % 8 of the 64-wide step;
-  // scale (row tid / 2 + 128 i, block tid % 2)
-  const int sr = tid >> 3, sc = (tid & 7) * 8;
-  const uint16_t* a0 = a.A + sc;
-  const uint16_t* w0 = a.W + (size_t)(n0 + sr) * K + sc;
-  const float* dp = a.D + (size_t)(n0 + (tid >> 1)) * (K / 32) + (tid & 1);
-  u32x4 rh[4], rl[4], rw[WI];
-  float rd[DI];
-  auto fetch = [&](int k0) __attribute__((always_inline)) {
+  const int fm = (Lp / (GROUP * NT)) * GROUP, gm = min(MT - fm, GROUP);
+  const int m0 = (fm + (Lp % (GROUP * NT)) % gm) * BM, n0 = ((Lp % (GROUP * NT)) / gm) * BN;
+  const int ns = KB / a.ks, kb0 = kz * ns;   // this block's K slice: 32-blocks [kb0, kb0 + ns)
+  const int rows = min(BM, M - m0);
+  const uint32_t arow = (uint32_t)KB * 128;
+  const int t0 = n0 / 16 + wv * NJ;          // this wave's first 16-row weight tile
+  const auto ra = buf_rsrc((const uint8_t*)a.A + (size_t)m0 * arow, (size_t)rows * arow);
+  const auto rw = buf_rsrc(a.W + (size_t)t0 * KB * 512, (size_t)NJ * KB * 1024);
+  const auto rs = buf_rsrc(a.D + (size_t)t0 * KB * 16, (size_t)NJ * KB * 64);
+  // staging: chunk tid + 256 i of a step is 16-byte unit q % 8 of row q / 8
+  uint32_t ga[AC], la[AC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint16_t* ar = a0 + (size_t)min(m0 + sr + 32 * i, M - 1) * K + k0;
-      rh[i] = *(const u32x4*)ar;
-      rl[i] = *(const u32x4*)(ar + MK);
-    }
+  for (int i = 0; i < AC; ++i) {
+    const int q = tid + 256 * i, row = q >> 3, c = q & 7;
+    ga[i] = (uint32_t)row * arow + c * 16;
+    la[i] = (row >> 4) * 2048 + c * 256 + (((row & 15) ^ c) * 16);
+  }
+  u32x4 ar[PA][AC], w[SL][NJ];
+  float d[SL][NJ];
+  // loads past the slice's end repeat its last step (never used)
+  auto load_a = [&](int sl, int s) __attribute__((always_inline)) {
+    const uint32_t so = (uint32_t)(kb0 + min(s, ns - 1)) * 128u;
 #pragma unroll
-    for (int i = 0; i < WI; ++i)
-      if (BN >= 32 * (i + 1) || sr + 32 * i < BN) rw[i] = *(const u32x4*)(w0 + (size_t)(32 * i) * K + k0);
-#pragma unroll
-    for (int i = 0; i < DI; ++i)
-      if (BN >= 128 * (i + 1) || tid + 256 * i < 2 * BN) rd[i] = dp[(size_t)(128 * i) * (K / 32) + k0 / 32];
+    for (int i = 0; i < AC; ++i) ar[sl][i] = buf_load16(ra, ga[i], so);
   };
-  auto stage = [&]() __attribute__((always_inline)) {
+  auto store_a = [&](int sl, int st) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = (sr + 32 * i) * kGBP + sc;
-      *(u32x4*)&Ah[r] = rh[i];
-      *(u32x4*)&Al[r] = rl[i];
-    }
+    for (int i = 0; i < AC; ++i) *(u32x4*)&As[st][la[i]] = ar[sl][i];
+  };
+  auto load_w = [&](int sl, int s) __attribute__((always_inline)) {
+    const int k = kb0 + min(s, ns - 1);
 #pragma unroll
-    for (int i = 0; i < WI; ++i)
-      if (BN >= 32 * (i + 1) || sr + 32 * i < BN) *(u32x4*)&Ws[(sr + 32 * i) * kGBP + sc] = rw[i];
+    for (int j = 0; j < NJ; ++j) w[sl][j] = buf_load16(rw, lane * 16, (uint32_t)(j * KB + k) * 1024u);
 #pragma unroll
-    for (int i = 0; i < DI; ++i)
-      if (BN >= 128 * (i + 1) || tid + 256 * i < 2 * BN) Ds[tid + 256 * i] = rd[i];
+    for (int j = 0; j < NJ; ++j)
+      d[sl][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, r16 * 4, (uint32_t)(j * KB + k) * 64u, 0));
   };
 
-  f32x4 acc[NI][NJ];
+  f32x4 acc[MI][NJ];
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int kb = kz * kn, ke = kb + kn;
-  fetch(kb);
-  for (int k0 = kb; k0 < ke; k0 += 64) {
-    __syncthreads();   // the previous step's LDS reads are done
-    stage();
-    __syncthreads();
-    if (k0 + 64 < ke) fetch(k0 + 64);
-    // the MFMA phase runs at raised wave priority: with two blocks on a CU
-    // the one computing issues ahead of the one staging (down 97 -> 85 us,
-    // O 24.3 -> 22.2 us at the 1B prefill shapes; no effect alone on a CU)
+  const int rdh = g * 256 + ((r16 ^ g) * 16), rdl = 1024 + g * 256 + ((r16 ^ (4 + g)) * 16);
+  load_a(0, 0);
+#pragma unroll
+  for (int p = 0; p < PW; ++p) load_w(p, p);
+  store_a(0, 0);
+#pragma unroll
+  for (int q = 0; q < PA; ++q) load_a((1 + q) % PA, 1 + q);
+  __syncthreads();
+  // step s, u = s mod the unroll: stage s + 1 of A goes to LDS and the loads
+  // of later steps go out, then this step's products
+  auto step = [&](int s, int u) __attribute__((always_inline)) {
+    const int sl = u % SL, st = u & 1;
+    store_a((u + 1) % PA, st ^ 1);
+    load_w((sl + PW) % SL, s + PW);
+    load_a((u + 1) % PA, s + 1 + PA);
+    // the MFMA phase runs at raised wave priority: of the waves on a SIMD the
+    // computing one issues ahead of the staging ones
     __builtin_amdgcn_s_setprio(1);
+    f32x4 p[2][NJ];
+    bf16x8 xh[2], xl[2];
+    auto read = [&](int i) __attribute__((always_inline)) {
+      xh[i & 1] = __builtin_bit_cast(bf16x8, *(const u32x4*)&As[st][i * 2048 + rdh]);
+      xl[i & 1] = __builtin_bit_cast(bf16x8, *(const u32x4*)&As[st][i * 2048 + rdl]);
+    };
+    auto scale = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      bf16x8 xh[NI], xl[NI], w[NJ];
-      float d[NJ];
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int o = (wm + 16 * i + c16) * kGBP + 32 * b + 8 * g;
-        xh[i] = lds_bf16x8(&Ah[o]);
-        xl[i] = lds_bf16x8(&Al[o]);
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(d[sl][j], p[i & 1][j][r], acc[i][j][r]);
+    };
+    // the schedule: a row tile's operands are read while the previous row
+    // tile multiplies, and its scale FMAs fill the issue slots between the
+    // next tile's MFMAs, two behind each
+    read(0);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      if (i + 1 < MI) read(i + 1);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        p[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh[i & 1], __builtin_bit_cast(bf16x8, w[sl][j]),
+                                                              f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        p[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl[i & 1], __builtin_bit_cast(bf16x8, w[sl][j]),
+                                                              p[i & 1][j], 0, 0, 0);
+      if (i > 0) scale(i - 1);
+      if (i == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);       // LDS reads
+      if (i + 1 < MI) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+      for (int q = 0; q < 2 * NJ; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                   // MFMA
+        if (i > 0) __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);        // VALU
       }
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        w[j] = lds_bf16x8(&Ws[(wn + 16 * j + c16) * kGBP + 32 * b + 8 * g]);
-        d[j] = Ds[(wn + 16 * j + c16) * 2 + b];
-      }
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh[i], w[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl[i], w[j], p, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(d[j], p[r], acc[i][j][r]);
-        }
     }
+    scale(MI - 1);
     __builtin_amdgcn_s_setprio(0);
+    __syncthreads();
+  };
+  constexpr int U = SL % 2 == 0 ? SL : 2 * SL;
+  static_assert(U % PA == 0, "the A registers rotate with the unroll");
+  for (int s = 0; s < ns; s += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u > 0 && s + u >= ns) break;
+      step(s + u, u);
+    }
   }
-  // D[i][j] of a 16x16 tile: lane l, register r -> row 4 (l / 16) + r, col l % 16
-  const size_t half_plane = (size_t)M * (a.N / 2);
+
+  // D of a 16x16 tile: lane l, register r -> row 4 (l / 16) + r, col l % 16
+  if (EPI == EPI_OUT) {
+    const auto rc = buf_rsrc(a.C + ((size_t)kz * M + m0) * N, (size_t)rows * N * 4);
+    const uint32_t vo = ((uint32_t)(4 * g) * N + n0 + wv * 16 * NJ + r16) * 4u;
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wm + 16 * i + 4 * g + r;
-      if (m >= M) continue;
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t v = vo + (uint32_t)(16 * i + r) * N * 4u;   // the checked part of the address
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int n = n0 + wn + 16 * j + c16;
-        if (EPI == EPI_OUT) {
-          a.C[(size_t)kz * M * a.N + (size_t)m * a.N + n] = acc[i][j][r];
-        } else if ((j & 1) == 0) {
-          // 16 gate rows (tile j), then their 16 up rows (tile j + 1)
-          const size_t o = (size_t)m * (a.N / 2) + (n >> 5) * 16 + (n & 15);
-          split_bf16(gelu_mul(acc[i][j][r], acc[i][j | 1][r]), &a.act[o], &a.act[half_plane + o]);
+        for (int j = 0; j < NJ; ++j)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r]), rc, v + 64 * j, 0, 0);
+      }
+  } else {
+    // 16 gate rows (tile j), then their 16 up rows (tile j + 1): 16 features
+    // per pair, two pairs per 32-block of the output rows (2 N bytes each)
+    const auto ro = buf_rsrc(a.act + (size_t)m0 * N, (size_t)rows * N * 2);
+    const int f0 = (n0 + wv * 16 * NJ) / 2;   // this wave's first feature
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t vo = (uint32_t)(16 * i + 4 * g + r) * N * 2u + (f0 >> 5) * 128u + r16 * 4u;
+        if (NJ % 4 == 0) {
+#pragma unroll
+          for (int j = 0; j < NJ; j += 4) {
+            uint32_t hi, lo;
+            split2_bf16(gelu_mul(acc[i][j][r], acc[i][(j + 1) % NJ][r]),
+                        gelu_mul(acc[i][(j + 2) % NJ][r], acc[i][(j + 3) % NJ][r]), hi, lo);
+            __builtin_amdgcn_raw_buffer_store_b32(hi, ro, vo + 32 * j, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(lo, ro, vo + 32 * j + 64, 0, 0);
+          }
+        } else {   // one pair: the low or high half of each dword
+          uint16_t hi, lo;
+          split_bf16(gelu_mul(acc[i][0][r], acc[i][1 % NJ][r]), &hi, &lo);
+          const uint32_t vh = vo + (f0 & 16) / 8;
+          __builtin_amdgcn_raw_buffer_store_b16(hi, ro, vh, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b16(lo, ro, vh + 64, 0, 0);
         }
       }
-    }
+  }
 }
+
+// Offset of element e of an A row: 32-blocks of hi then lo.
+__device__ __forceinline__ int a_slot(int e) { return ((e >> 5) << 6) + (e & 31); }
 
 // Row kernels (one block per prompt row, H <= 2048).
 __device__ __forceinline__ void row_norm_out(const float* r, const float* w, int H, float eps, uint16_t* out,
-                                             size_t plane, float* sh4, int n) {
+                                             float* sh4, int n) {
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i)
@@ -1413,7 +1487,7 @@ __device__ __forceinline__ void row_norm_out(const float* r, const float* w, int
   for (int i = 0; i < 8; ++i)
     if (i < n) {
       const int e = threadIdx.x + 256 * i;
-      split_bf16((r[i] * w[e]) * ri, &out[e], &out[plane + e]);
+      split_bf16((r[i] * w[e]) * ri, &out[a_slot(e)], &out[a_slot(e) + 32]);
     }
 }
 
@@ -1433,7 +1507,7 @@ __global__ __launch_bounds__(256) void k_rows_embed(RowArgs a) {
       h[i] = embed_elem(g, token, tid + 256 * i);
       a.res_out[(size_t)row * H + tid + 256 * i] = h[i];
     }
-  row_norm_out(h, a.w_pre, H, a.eps, a.x_out + (size_t)row * H, (size_t)a.M * H, sh4, n);
+  row_norm_out(h, a.w_pre, H, a.eps, a.x_out + (size_t)row * H * 2, sh4, n);
 }
 
 __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
@@ -1503,7 +1577,6 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
     }
   }
   const float ri = rsq(wave_sum_dpp(ss) / (float)H + a.eps);
-  const size_t plane = (size_t)a.M * H;
 #pragma unroll
   for (int k = 0; k < KF; ++k) {
     const int f = lane + 64 * k;
@@ -1513,9 +1586,9 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
       uint16_t hi[4], lo[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) split_bf16(y[j], &hi[j], &lo[j]);
-      const size_t e = (size_t)row * H + 4 * f;
-      *(uint2*)(a.x_out + e) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-      *(uint2*)(a.x_out + plane + e) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
+      uint16_t* xo = a.x_out + (size_t)row * H * 2 + a_slot(4 * f);
+      *(uint2*)xo = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
+      *(uint2*)(xo + 32) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
     }
   }
 }
@@ -1711,10 +1784,13 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t* __restrict__ src
 // GGUF Q8_0 rows -> the prefill GEMM's weights: int8 values as bf16 (exact)
 // and fp32 block scales, one thread per 32-block. Source row r goes to row
 // r + off, or with half = 16 to (r / 16) * 32 + r % 16 + off (gate / up
-// groups of 16 + 16 rows).
+// groups of 16 + 16 rows). The 16 rows of tile t and the 32 inputs of block b
+// are the 1 KB at ((t nb) + b) * 1 KB: lane l of the MFMA operand holds row
+// l % 16, inputs 8 (l / 16) .. + 7; their scales are 16 floats at t nb + b.
+// act_order: inputs in the GeGLU epilogue's order (the down matrix).
 __global__ __launch_bounds__(256) void k_q8_bf16(const uint8_t* __restrict__ src, uint16_t* __restrict__ wb,
                                                  float* __restrict__ wd, long long rows, int K, long long off,
-                                                 int half) {
+                                                 int half, int act_order) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   const int nb = K / 32;
   if (idx >= rows * nb) return;
@@ -1722,12 +1798,14 @@ __global__ __launch_bounds__(256) void k_q8_bf16(const uint8_t* __restrict__ src
   const int b = (int)(idx - r * nb);
   const long long R = half > 0 ? (r / half) * 2 * half + r % half + off : r + off;
   const uint8_t* blk = src + (size_t)idx * 34;
-  wd[R * nb + b] = (float)__builtin_bit_cast(_Float16, (uint16_t)(blk[0] | (blk[1] << 8)));
-  uint32_t* o = (uint32_t*)(wb + R * K + 32 * b);
+  const long long tb = (R >> 4) * nb + b;
+  const int r16 = (int)(R & 15);
+  wd[tb * 16 + r16] = (float)__builtin_bit_cast(_Float16, (uint16_t)(blk[0] | (blk[1] << 8)));
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const float f0 = (float)(int8_t)blk[2 + 2 * j], f1 = (float)(int8_t)blk[3 + 2 * j];
-    o[j] = (__float_as_uint(f0) >> 16) | (__float_as_uint(f1) & 0xffff0000u);
+  for (int f = 0; f < 32; ++f) {
+    const int p = act_order ? act_slot(f) : f;
+    wb[tb * 512 + ((p >> 3) * 16 + r16) * 8 + (p & 7)] =
+        (uint16_t)(__float_as_uint((float)(int8_t)blk[2 + f]) >> 16);
   }
 }
 
@@ -1935,12 +2013,12 @@ int launch_class_major(const uint8_t* src, uint8_t* dst, long long rows, int Kp,
 }
 
 int launch_q8_bf16(const uint8_t* src, uint16_t* wb, float* wd, long long rows, int K, long long off, int half,
-                   void* stream) {
+                   int act_order, void* stream) {
   if (K % 32 || off < 0 || (half != 0 && half != 16)) return (int)hipErrorInvalidValue;
   const long long total = rows * (K / 32);
   if (total <= 0) return 0;
   hipLaunchKernelGGL(k_q8_bf16, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, src, wb,
-                     wd, rows, K, off, half);
+                     wd, rows, K, off, half, act_order);
   return (int)hipGetLastError();
 }
 
@@ -1951,18 +2029,38 @@ int launch_dequant(const uint8_t* src, float* out, long long n, void* stream) {
   return (int)hipGetLastError();
 }
 
+template <int EPI, int MI, int NJ, int PW, int PA, int OCC>
+static int launch_gemm_t(const GemmArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((k_gemm<EPI, MI, NJ, PW, PA, OCC>), dim3(a.N / (64 * NJ), (a.M + 16 * MI - 1) / (16 * MI), a.ks),
+                     dim3(256), 0, s, a);
+  return (int)hipGetLastError();
+}
+
 int launch_gemm(int epi, const GemmArgs& a, void* stream) {
-  const int bn = a.bn;
-  if (a.M < 1 || (bn != 128 && bn != 144 && bn != 96) || (bn != 128 && epi != EPI_OUT) || a.N < bn || a.N % bn ||
-      a.K < 64 || a.ks < 1 || a.ks > kGemmMaxSlices || a.K % (64 * a.ks) || !a.A || !a.W || !a.D ||
+  if (a.tile < 0 || a.tile >= GT_COUNT) return (int)hipErrorInvalidValue;
+  const GemmTile& t = kGemmTiles[a.tile];
+  if (a.M < 1 || a.N < 64 || a.N % (64 * t.nj) || !(epi == EPI_OUT ? t.out : t.geglu) || a.K < 64 || a.ks < 1 ||
+      a.ks > kGemmMaxSlices || a.K % (32 * a.ks) || !a.A || !a.W || !a.D ||
       (epi == EPI_OUT ? !a.C : (!a.act || a.ks != 1)))
     return (int)hipErrorInvalidValue;
-  dim3 grid(a.N / bn, (a.M + kGBM - 1) / kGBM, a.ks);
-  if (epi == EPI_GEGLU) hipLaunchKernelGGL((k_gemm<EPI_GEGLU, 4, 4>), grid, dim3(256), 0, (hipStream_t)stream, a);
-  else if (bn == 128) hipLaunchKernelGGL((k_gemm<EPI_OUT, 4, 4>), grid, dim3(256), 0, (hipStream_t)stream, a);
-  else if (bn == 96) hipLaunchKernelGGL((k_gemm<EPI_OUT, 4, 3>), grid, dim3(256), 0, (hipStream_t)stream, a);
-  else hipLaunchKernelGGL((k_gemm<EPI_OUT, 2, 9>), grid, dim3(256), 0, (hipStream_t)stream, a);
-  return (int)hipGetLastError();
+  hipStream_t s = (hipStream_t)stream;
+  if (epi == EPI_GEGLU) {
+    switch (a.tile) {
+      case GT_32x128: return launch_gemm_t<EPI_GEGLU, 2, 2, 3, 2, 4>(a, s);
+      case GT_64x128: return launch_gemm_t<EPI_GEGLU, 4, 2, 3, 2, 3>(a, s);
+      case GT_64x256: return launch_gemm_t<EPI_GEGLU, 4, 4, 1, 1, 3>(a, s);
+      case GT_128x256: return launch_gemm_t<EPI_GEGLU, 8, 4, 1, 1, 2>(a, s);
+    }
+  } else {
+    switch (a.tile) {
+      case GT_32x64: return launch_gemm_t<EPI_OUT, 2, 1, 3, 2, 4>(a, s);
+      case GT_32x128: return launch_gemm_t<EPI_OUT, 2, 2, 3, 2, 4>(a, s);
+      case GT_32x192: return launch_gemm_t<EPI_OUT, 2, 3, 3, 2, 3>(a, s);
+      case GT_64x128: return launch_gemm_t<EPI_OUT, 4, 2, 3, 2, 3>(a, s);
+      case GT_64x192: return launch_gemm_t<EPI_OUT, 4, 3, 2, 1, 3>(a, s);
+    }
+  }
+  return (int)hipErrorInvalidValue;
 }
 
 int launch_rows_embed(const RowArgs& a, void* stream) {
@@ -1980,7 +2078,7 @@ int launch_rows_resid(const RowArgs& a, void* stream) {
 
 int launch_rows_kv(const RowArgs& a, void* stream) {
   if (a.M < 1) return (int)hipErrorInvalidValue;
-  if (a.n_q < 1 || a.n_q > kAttnMaxQ || a.pre_planes > kQkvMaxSlices ||
+  if (a.n_q < 1 || a.n_q > kAttnMaxQ || a.pre_planes > kGemmMaxSlices ||
       (a.pre_planes > 1 && a.pre_stride < (size_t)a.M * (a.n_q + 2) * kHeadDim))
     return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(k_rows_kv, dim3(a.M), dim3(64 * (a.n_q + 1)), 0, (hipStream_t)stream, a);

@@ -40,8 +40,8 @@ struct Layer {
   uint8_t* o = nullptr;
   uint8_t* gu = nullptr;    // gate/up rows interleaved GR/2 + GR/2 per row group
   uint8_t* down = nullptr;
-  // batched prefill GEMM weights (prefill_batch > 0): int8 values as bf16
-  // [N][K] and fp32 block scales [N][K / 32]; gate / up in groups of 16 + 16
+  // batched prefill GEMM weights (prefill_batch > 0): int8 values as bf16 and
+  // fp32 block scales in MFMA operand order; gate / up in groups of 16 + 16
   uint16_t *qkv_b = nullptr, *o_b = nullptr, *gu_b = nullptr, *down_b = nullptr;
   float *qkv_d = nullptr, *o_d = nullptr, *gu_d = nullptr, *down_d = nullptr;
   float* norm[N_NNORM] = {};
@@ -119,7 +119,7 @@ struct gg_ctx {
   // batched prefill (prefill_batch > 0)
   int pf_M = 0;
   float *pf_hidden = nullptr, *pf_residual = nullptr, *pf_qkv = nullptr, *pf_o = nullptr, *pf_part = nullptr;
-  // GEMM inputs as bf16 hi / lo planes (the slice's M rows each)
+  // GEMM inputs as bf16 hi / lo (the slice's M rows each)
   uint16_t *pf_xn = nullptr, *pf_attn = nullptr, *pf_act = nullptr;
 
   // pinned host mirrors
@@ -638,35 +638,32 @@ int sync(gg_ctx* c, const char* what) {
 }
 
 
-// Block tile width (128, or 144 or 96 for a C output whose width it divides)
-// and K slices (up to max_ks, dividing K into whole 64-steps) that minimise
-// the modelled time, in units of one block's 64-wide step on a CU of its own:
-// steps per block times the load of the busiest CU, where n >= 2 co-resident
-// blocks take 0.75 n of one block's time (measured on the 1B down GEMM: 144
-// blocks x 108 steps 165 us, 288 x 54 124 us), times 1.2 for the 144-wide
-// tile (1.125x the work per step; 85.5 us for 512 x 27 steps against 98.6 us
-// for 432 x 36 steps of the 128-wide tile) or 0.96 for the 96-wide one (the
-// 1B QKV GEMM, two blocks on the busiest CUs either way: 512 x 9 steps 24.7
-// us against 384 x 9 steps 25.7 us), plus one unit per 2.29 M outputs of each
-// slice for the consumer's read of that slice (9.4 MB in ~1.9 us at M = 2048,
-// N = 1152). C must hold that many slices; the consumer adds them.
-void gemm_plan(int N, int K, int M, int max_ks, bool out, int* bn_out, int* ks_out) {
-  const int steps = K / 64;
-  double best_cost = 0.0;
-  *bn_out = 128;
-  *ks_out = 1;
-  for (int bn : {128, 144, 96}) {
-    if (N % bn || (bn != 128 && !out)) continue;
-    const int tiles = (N / bn) * ((M + 127) / 128);
+// Block tile and K slices (up to max_ks, dividing K into whole 32-blocks)
+// that minimise the modelled time: the 32-wide steps of a block times the
+// fitted time of a step with as many blocks on the CU as this launch puts
+// there (kGemmTiles; 0.3 of the round-up to whole blocks per CU counts, the
+// rest overlaps), plus 8 bytes per output of each slice at 5 TB/s for writing
+// it and for the consumer's read. Over the timings that the fit used, the
+// choice is 4% slower than the best tile and split on average and 21% at
+// worst, while the best fixed tile of a matrix is off by 2x at the ends.
+void gemm_plan(GemmArgs& g, int max_ks, bool out) {
+  const int steps = g.K / 32;
+  double best = 0.0;
+  g.tile = -1;
+  for (int t = 0; t < GT_COUNT; ++t) {
+    const GemmTile& T = kGemmTiles[t];
+    if (g.N % (64 * T.nj) || !(out ? T.out : T.geglu)) continue;
+    const int tiles = (g.N / (64 * T.nj)) * cdiv(g.M, 16 * T.mi);
     for (int ks = 1; ks <= max_ks; ++ks) {
       if (steps % ks) continue;
-      const int per_cu = (tiles * ks + 255) / 256;
-      const double cost = (per_cu == 1 ? 1.0 : 0.75 * per_cu) * (steps / ks) * (bn == 144 ? 1.2 : bn == 96 ? 0.96 : 1.0) +
-                          (out ? ks * ((double)M * N / 2.29e6) : 0.0);
-      if ((bn == 128 && ks == 1) || cost < best_cost) {
-        best_cost = cost;
-        *bn_out = bn;
-        *ks_out = ks;
+      const double blocks = (double)tiles * ks;
+      const double per_cu = 0.7 * std::max(1.0, blocks / 256) + 0.3 * std::ceil(blocks / 256);
+      const double cost = (steps / ks) * (T.lat + T.thr * (per_cu - 1.0)) +
+                          (out ? ks * ((double)g.M * g.N * 8 / 5e6) : 0.0);
+      if (g.tile < 0 || cost < best) {
+        best = cost;
+        g.tile = t;
+        g.ks = ks;
       }
     }
   }
@@ -683,7 +680,7 @@ GemmArgs gemm_base(const uint16_t* A, const uint16_t* W, const float* D, int N, 
   g.K = K;
   g.C = C;
   g.act = act;
-  gemm_plan(N, K, M, C ? max_ks : 1, C != nullptr, &g.bn, &g.ks);
+  gemm_plan(g, C ? max_ks : 1, C != nullptr);
   return g;
 }
 
@@ -709,7 +706,7 @@ int prefill_slice(gg_ctx* c, const int32_t* d_tokens, int M, int start) {
   for (int l = 0; l < c->L; ++l) {
     Layer& Ly = c->layers[l];
     const bool swa = is_swa(c->c, l);
-    const GemmArgs gq = gemm_base(c->pf_xn, Ly.qkv_b, Ly.qkv_d, c->NQKV, c->H, M, c->pf_qkv, nullptr, kQkvMaxSlices);
+    const GemmArgs gq = gemm_base(c->pf_xn, Ly.qkv_b, Ly.qkv_d, c->NQKV, c->H, M, c->pf_qkv, nullptr, qkv_slices(M));
     GG_TRY(launch_rc(c, launch_gemm(EPI_OUT, gq, s), "prefill qkv"));
     RowArgs kv{};
     kv.M = M;
@@ -738,7 +735,7 @@ int prefill_slice(gg_ctx* c, const int32_t* d_tokens, int M, int start) {
     at.pf_rows = M;
     at.pf_chunk = prefill_chunk(at.window, start, M);
     GG_TRY(launch_rc(c, launch_prefill_attention(at, M, s), "prefill attention"));
-    const GemmArgs go = gemm_base(c->pf_attn, Ly.o_b, Ly.o_d, c->H, c->QD, M, c->pf_o, nullptr, kGemmMaxSlices);
+    const GemmArgs go = gemm_base(c->pf_attn, Ly.o_b, Ly.o_d, c->H, c->QD, M, c->pf_o, nullptr, gemm_slices(M));
     GG_TRY(launch_rc(c, launch_gemm(EPI_OUT, go, s), "prefill o"));
     RowArgs r1 = r;
     r1.pre = c->pf_o;
@@ -751,7 +748,7 @@ int prefill_slice(gg_ctx* c, const int32_t* d_tokens, int M, int start) {
     r1.x_out = c->pf_xn;
     GG_TRY(launch_rc(c, launch_rows_resid(r1, s), "prefill post-attn"));
     GG_TRY(launch_rc(c, launch_gemm(EPI_GEGLU, gemm_base(c->pf_xn, Ly.gu_b, Ly.gu_d, 2 * c->I, c->H, M, nullptr, c->pf_act), s), "prefill gate/up"));
-    const GemmArgs gd = gemm_base(c->pf_act, Ly.down_b, Ly.down_d, c->H, c->I, M, c->pf_o, nullptr, kGemmMaxSlices);
+    const GemmArgs gd = gemm_base(c->pf_act, Ly.down_b, Ly.down_d, c->H, c->I, M, c->pf_o, nullptr, gemm_slices(M));
     GG_TRY(launch_rc(c, launch_gemm(EPI_OUT, gd, s), "prefill down"));
     if (l + 1 < c->L) {
       RowArgs r2 = r;
@@ -991,7 +988,7 @@ int gg_upload_tensor(gg_ctx* c, const char* name, uint32_t type, const uint64_t*
       case Q_DOWN: wb = Ly.down_b; wd = Ly.down_d; break;
       default: break;
     }
-    GG_TRY(launch_rc(c, launch_q8_bf16(c->staging, wb, wd, rows, (int)K, boff, bhalf, c->stream), "prefill weights"));
+    GG_TRY(launch_rc(c, launch_q8_bf16(c->staging, wb, wd, rows, (int)K, boff, bhalf, bit == Q_DOWN, c->stream), "prefill weights"));
   }
   GG_TRY(sync(c, "repack"));
   if (layer < 0) c->have_embd = true;
@@ -1054,9 +1051,11 @@ int gg_finalize(gg_ctx* c) {
     const size_t MH = (size_t)M * c->H * 4;
     GG_TRY(dalloc(c, &c->pf_hidden, MH));
     GG_TRY(dalloc(c, &c->pf_residual, MH));
-    GG_TRY(dalloc(c, &c->pf_xn, MH));   // bf16 hi + lo planes: 4 bytes per element
-    GG_TRY(dalloc(c, &c->pf_o, kGemmMaxSlices * MH));   // K slices of the O / down GEMMs
-    GG_TRY(dalloc(c, &c->pf_qkv, (size_t)kQkvMaxSlices * M * c->NQKV * 4));   // K slices of the QKV GEMM
+    GG_TRY(dalloc(c, &c->pf_xn, MH));   // bf16 hi + lo: 4 bytes per element
+    // K slices of the O / down and QKV GEMMs: M rows, or fewer rows in more slices
+    const int few = std::min(M, kGemmFewRows);
+    GG_TRY(dalloc(c, &c->pf_o, (size_t)std::max(gemm_slices(M) * M, gemm_slices(few) * few) * c->H * 4));
+    GG_TRY(dalloc(c, &c->pf_qkv, (size_t)std::max(qkv_slices(M) * M, qkv_slices(few) * few) * c->NQKV * 4));
     GG_TRY(dalloc(c, &c->pf_attn, (size_t)M * c->QD * 4));
     GG_TRY(dalloc(c, &c->pf_act, (size_t)M * c->I * 4));
     GG_TRY(dalloc(c, &c->pf_part, (size_t)M * kPrefillChunks * kAttnMaxQ * (2 + kHeadDim) * 4));
