@@ -141,12 +141,19 @@ struct AttnArgs {
   uint16_t* pf_out;        // batched prefill: the O GEMM's input, [row][n_q * 8][2][32]
   float* q_dbg;            // decode, optional: normed+roped q of this token
   // batched prefill: prompt row r sits at position pf_start + r; q of every
-  // row is already normed + roped in `qkv`, K/V of every position are in the
-  // cache; keys of a 16-row query tile are split in chunks of pf_chunk
+  // row and k, v of every position that the slice attends to are in operand
+  // order (k_rows_kv); the key tiles of a 32-row query tile are split in
+  // chunks of pf_chunk
   int pf_start;
   int pf_rows;
   int pf_chunk;
+  const uint16_t* q_frag;
+  const uint8_t* kv_planes;
 };
+// q in MFMA operand order: [row / 16][n_q][8 dim blocks of 32][hi, lo][64 lanes][8]. k and v of 32 keys:
+// K [8 dim blocks][2 key tiles][hi, lo][64][8], then V [16 dim tiles][hi, lo][64][8] (tile 2 k + e, column c:
+// dim 32 k + 2 c + e).
+constexpr size_t kKvTileBytes = 65536;
 
 // Prefill GEMM on bf16 MFMA: C[M x N] = A[M x K] * W[N x K]^T. A comes as
 // bf16 hi / lo (hi = bf16(x), lo = bf16(x - hi)), a row's 32-blocks one after
@@ -183,7 +190,7 @@ struct RowArgs {
   float* res_out;          // [M][H] new residual stream
   uint16_t* x_out;         // normed GEMM input, [M][H / 32][2][32]
   float* last_hidden;      // optional: row M-1 of res_out (per-layer history)
-  // KV: k/v of each row into the cache, q heads normed + roped in place
+  // KV: k/v of each row into the cache, q / k / v in operand order
   const float* qkv;
   int n_q;
   const float* q_norm;
@@ -191,6 +198,10 @@ struct RowArgs {
   const float* rope;
   float* k_cache;
   float* v_cache;
+  int kv_lo;               // first key position that the slice's attention reads
+  float q_scale;           // log2(e) / sqrt(head_dim): scores in log2 units
+  uint16_t* q_frag;
+  uint8_t* kv_planes;
 };
 
 struct FinalArgs {
@@ -362,23 +373,35 @@ constexpr GemmTile kGemmTiles[GT_COUNT] = {
     {4, 2, true, true, .361f, .355f},  {4, 3, true, false, .463f, .473f}, {4, 4, false, true, .605f, .485f},
     {8, 4, false, true, .955f, .919f}};
 constexpr int kGemmMaxSlices = 8;   // K slices of a prefill GEMM (summed by the consumer)
+constexpr int kQkvMaxSlices = 4;    // ... of the QKV GEMM (summed by k_rows_kv)
 // Slices that the output buffers of an M-row GEMM hold: few rows need more
 // blocks and their slices are small.
 constexpr int kGemmFewRows = 512;
 inline int gemm_slices(int M) { return M <= kGemmFewRows ? kGemmMaxSlices : 4; }   // O, down
-inline int qkv_slices(int M) { return M <= kGemmFewRows ? 4 : 2; }
+inline int qkv_slices(int M) { return M <= kGemmFewRows ? kQkvMaxSlices : 2; }
 constexpr int kPrefillChunks = 16;   // key chunks per query tile in the batched prefill attention
-constexpr int kPrefillMinChunk = 160;
-// Longest key span of a 32-row query tile of a prefill of M rows at `start`.
-inline int prefill_max_span(int window, int start, int M) {
-  const int full = start + M;
-  return window > 0 && window + 31 < full ? window + 31 : full;
+// Most 32-key tiles that a 32-row query tile of a prefill of M rows at `start` reads.
+inline int prefill_max_tiles(int window, int start, int M) {
+  const int full = (start + M + 31) / 32;
+  return window > 0 ? (full < (window + 31 + 31) / 32 + 1 ? full : (window + 31 + 31) / 32 + 1) : full;
 }
-// Keys per chunk: a multiple of 32, >= kPrefillMinChunk, at most kPrefillChunks chunks.
+// Key tiles per chunk: the split (at most kPrefillChunks chunks) with the
+// least modelled time, in tiles of a block on a CU of its own (2 us): rounds
+// of 256 blocks times a chunk's tiles and 2 for its start and end, plus the
+// merge of several chunks (a launch, and the partials written and read).
 inline int prefill_chunk(int window, int start, int M) {
-  const int span = prefill_max_span(window, start, M);
-  const int c = 32 * ((span + 32 * kPrefillChunks - 1) / (32 * kPrefillChunks));
-  return c > kPrefillMinChunk ? c : kPrefillMinChunk;
+  const int tiles = prefill_max_tiles(window, start, M), qt = (M + 31) / 32;
+  int best = tiles;
+  double best_cost = 0.0;
+  for (int n = 1; n <= kPrefillChunks && n <= tiles; ++n) {
+    const int ct = (tiles + n - 1) / n, nc = (tiles + ct - 1) / ct;
+    const double cost = (double)((qt * nc + 255) / 256) * (ct + 2) + (nc > 1 ? 1.5 + nc * M * 4e-4 : 0.0);
+    if (n == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = ct;
+    }
+  }
+  return best;
 }
 
 }  // namespace gg

@@ -870,30 +870,33 @@ __global__ __launch_bounds__(256) void k_select2(SelectArgs a, int nb) {
 // one prompt token per decode pass, engine.ts:923-928, with the
 // scores / softmax / weighted V of shaders.ts:229-325).
 //
-// Block (x = key chunk, y = query tile) covers 32 prompt rows with 8 waves;
-// wave w computes query head w % 4 of rows 16 (w / 4) .. + 15 over the
-// chunk's keys, which are staged 32 rows at a time in LDS and shared by the
-// heads (one KV head) and both row halves, so each key's hi / lo split
-// serves 128 (row, head) pairs.
-//   S^T = K Q^T  on v_mfma_f32_16x16x32_bf16 with q and k split into bf16
-//                hi + lo (k and v when they are staged, q once per block):
-//                per 32 dims the products hi.hi, lo.hi and hi.lo, fp32
-//                accumulate (the dropped lo.lo term is below 2^-16 |k| |q|). Operand row
-//                c of key tile j (j < 2) is key 8 (c / 4) + 4 j + c % 4, so
-//                lane l holds S^T[key 8 g + 4 j + r][row l % 16] for r < 4,
-//                g = lane / 16.
+// k_rows_kv leaves q, k and v as bf16 hi / lo in MFMA operand order, so the
+// splits are made once per value and staging is a plain copy. Block (x = key
+// chunk, y = query tile) covers 32 prompt rows with four waves, one per query
+// head, on one wave's registers per SIMD: a wave holds its 32 rows' q (128
+// registers) and output (128), so every K and V operand read from LDS feeds
+// two row tiles; 16-row waves, two per SIMD, would read 170 bytes of LDS per
+// MFMA cycle of a CU, above its 128.
+//   S^T = K Q^T  on v_mfma_f32_16x16x32_bf16, q scaled by log2(e)/16 before
+//                its split: per 32 dims the products hi.hi, lo.hi and hi.lo,
+//                fp32 accumulate (the dropped lo.lo term is below 2^-16
+//                |k| |q|). Operand row c of key tile j (j < 2) is key
+//                8 (c / 4) + 4 j + c % 4, so lane l holds S^T[key 8 g + 4 j
+//                + r][row l % 16] for r < 4, g = lane / 16.
 //   O += P V     on v_mfma_f32_16x16x32_bf16, the same three products of
 //                bf16 hi + lo splits: A = P from lane l's own S^T registers
-//                (keys 8 g .. 8 g + 7 in order), B = V^T rows staged per
-//                dim; lane l holds O[row 4 g + r][16 i + l % 16] for i < 16.
-// Softmax statistics of row l % 16 stay online per lane: the max is reduced
-// over the four lane groups each tile, the sum once at the end. LDS rows are
-// unpadded and XOR-swizzled so that the ds_read_b128 operand reads (16 rows
-// per lane group) hit distinct banks: 16-byte unit u of K row k sits at
-// u ^ ((k % 4) + 4 (k / 8)), unit u (keys 8u .. 8u + 7) of V^T dim row d at
-// u ^ ((d / 2) % 4). A query tile whose span fits one chunk writes
-// O / l; otherwise every chunk leaves (m, l, O) in `part` for
-// k_attn_pf_merge.
+//                (keys 8 g .. 8 g + 7 in order), B = V^T per dim; tile 2 k +
+//                e column c is dim 32 k + 2 c + e, so lane l holds O[row
+//                4 g + r] of adjacent dims and stores them as one word.
+// Pipeline of 32-key tiles, one barrier each: while tile t's exponentials and
+// splits run in the issue slots between the MFMAs of tile t + 1's scores and
+// its P V follows, the next K and V tiles go to the other LDS stage by DMA
+// (64 KB per tile, two stages, no registers).
+// The softmax reference of a row (l % 16, per lane) moves only when a tile's
+// maximum exceeds it by more than 2^8, so O is rescaled rarely; every
+// probability is relative to the same reference until then, in fp32. A query
+// tile whose span fits one chunk writes O / l; otherwise every chunk leaves
+// (reference, l, O) in `part` for k_attn_pf_merge.
 // ---------------------------------------------------------------------------
 
 // x = hi + lo + e with hi = bf16(x), lo = bf16(x - hi), |e| <= 2^-17 |x|
@@ -938,252 +941,296 @@ __device__ __forceinline__ float pf_xor32_max(float v) {
 }
 
 constexpr int kPfRows = 32;   // query rows per block: two 16-row MFMA tiles
-__device__ __forceinline__ bf16x8 lds_bf16x8(const uint16_t* p) {
+__device__ __forceinline__ bf16x8 lds_bf16x8(const uint8_t* p) {
   return __builtin_bit_cast(bf16x8, *(const u32x4*)p);
 }
 
-constexpr int kPfKeys = 32;   // keys per LDS tile
+constexpr int kPfKeys = 32;                    // keys per tile
+constexpr int kPfTile = kPfKeys * 1024;        // bytes of a K (or V) tile: 256 dims, hi and lo
+static_assert(kKvTileBytes == 2 * kPfTile, "a tile of the planes is its K part, then its V part");
 
 __device__ __forceinline__ int pf_key_lo(const AttnArgs& a, int pos) {
   return a.window > 0 ? max(0, pos - a.window + 1) : 0;
 }
 
-// Keys of query tile qt (kPfRows rows): [lo(first row), last row], chunks of
-// pf_chunk keys.
-__device__ __forceinline__ void pf_tile_span(const AttnArgs& a, int qt, int* klo, int* khi, int* nkc) {
+// Key tiles [*t0, *t1] of query tile qt (kPfRows rows), in *nkc chunks of
+// pf_chunk tiles.
+__device__ __forceinline__ void pf_tile_span(const AttnArgs& a, int qt, int* t0, int* t1, int* nkc) {
   const int p_first = a.pf_start + qt * kPfRows;
   const int p_last = a.pf_start + min(qt * kPfRows + kPfRows - 1, a.pf_rows - 1);
-  *klo = pf_key_lo(a, p_first);
-  *khi = p_last;
-  *nkc = (p_last - *klo + a.pf_chunk) / a.pf_chunk;
+  *t0 = pf_key_lo(a, p_first) / kPfKeys;
+  *t1 = p_last / kPfKeys;
+  *nkc = (*t1 - *t0 + a.pf_chunk) / a.pf_chunk;
 }
 
-__global__ __launch_bounds__(512, 1) void k_attn_pf(AttnArgs a) {
-  __shared__ __align__(16) uint16_t Kh[kPfKeys * kHeadDim];
-  __shared__ __align__(16) uint16_t Kl[kPfKeys * kHeadDim];
-  __shared__ __align__(16) uint16_t Vh[kHeadDim * kPfKeys];   // V^T: [dim][key]
-  __shared__ __align__(16) uint16_t Vl[kHeadDim * kPfKeys];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = wv & 3, rt = wv >> 2;
+__global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
+  __shared__ __align__(16) uint8_t Ks[2][kPfTile];
+  __shared__ __align__(16) uint8_t Vs[2][kPfTile];
+  const int tid = threadIdx.x, lane = tid & 63, h = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
   const int M = a.pf_rows, nq = a.n_q, qt = blockIdx.y, kc = blockIdx.x;
-  int klo, khi, nkc;
-  pf_tile_span(a, qt, &klo, &khi, &nkc);
+  int t0, t1, nkc;
+  pf_tile_span(a, qt, &t0, &t1, &nkc);
   if (kc >= nkc) return;
-  const int k0 = klo + kc * a.pf_chunk, k1 = min(k0 + a.pf_chunk, khi + 1);
-  const bool active = h < nq;
+  const int tb = t0 + kc * a.pf_chunk, te = min(tb + a.pf_chunk, t1 + 1);   // key tiles [tb, te)
+  // staging: a K or V tile goes to LDS as it is, by DMA: wave w copies KBs
+  // 8 w .. 8 w + 7, each instruction one KB (lane l's 16 bytes to slot l of
+  // M0 + offset; the offset counts on both sides). Inline asm, because the
+  // compiler would wait for every DMA in flight before any LDS read; arrived()
+  // waits for them explicitly before the barrier that precedes their readers.
+  auto copy = [&](int t, int part, uint8_t* lds) __attribute__((always_inline)) {
+    const uint8_t* src = a.kv_planes + (size_t)t * kKvTileBytes + part * kPfTile + h * 8192;
+    const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + h * 8192;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+      asm volatile(
+          "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\t"
+          "global_load_lds_dwordx4 %1, %2 offset:2048\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072"
+          ::"s"(__builtin_amdgcn_readfirstlane(dst + half * 4096)), "v"(lane * 16), "s"(src + half * 4096)
+          : "memory", "m0");
+  };
+  auto arrived = []() __attribute__((always_inline)) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+  copy(tb, 0, Ks[0]);
+  copy(tb, 1, Vs[0]);
+  copy(min(tb + 1, te - 1), 0, Ks[1]);
 
-  // K staging: wave w moves key rows 8 i + w of a tile, lane = float4 slot.
-  // V of a tile is fetched while its scores run, K of the next tile while
-  // the weighted sum runs, so the two staging sets are never live together.
-  float4 st[4];
-  auto fetch = [&](const float* cache, int kt) {
+  // q of row tiles 2 qt + rt: [tile][head][t][plane][lane][8]; waves past the
+  // last head repeat it and write nothing
+  bf16x8 qh[2][8], ql[2][8];
+  const u32x4* qp = (const u32x4*)(a.q_frag + (size_t)(2 * qt * nq + min(h, nq - 1)) * 16 * kHeadDim * 2) + lane;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = kt + 8 * i + wv;
-      st[i] = *(const float4*)(cache + (size_t)(key < k1 ? key : k0) * kHeadDim + 4 * lane);
-      if (key >= k1) st[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  };
-  // K rows as bf16 hi / lo planes (hi = bf16(k), lo = bf16(k - hi)); the
-  // 16-byte unit u of row kr sits at u ^ kswz(kr), kswz = key bits 0, 1, 3, 4,
-  // so that the 16 rows of one MFMA operand read cover all 16 bank groups
-  auto kswz = [](int kr) { return (kr & 3) | ((kr >> 3) << 2); };
-  auto stage_k = [&]() {
+  for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int kr = 8 * i + wv;
-      const float4 x = st[i];
-      bf16x4 hi, lo;
-      split4_bf16(x.x, x.y, x.z, x.w, hi, lo);
-      const int o = kr * kHeadDim + 8 * ((lane >> 1) ^ kswz(kr)) + 4 * (lane & 1);
-      *(bf16x4*)&Kh[o] = hi;
-      *(bf16x4*)&Kl[o] = lo;
+    for (int t = 0; t < 8; ++t) {
+      qh[rt][t] = __builtin_bit_cast(bf16x8, qp[(size_t)rt * nq * 1024 + t * 128]);
+      ql[rt][t] = __builtin_bit_cast(bf16x8, qp[(size_t)rt * nq * 1024 + t * 128 + 64]);
     }
-  };
-  // V^T as bf16 hi / lo planes, 32 keys (64 bytes) per dim row; the 16-byte
-  // unit u (keys 8u .. 8u + 7) of dim row d sits at u ^ ((d / 2) % 4). Wave w
-  // fetches keys 4 w .. 4 w + 3, lane l dims 4 l .. 4 l + 3 (one 16-byte load
-  // per key), and writes half w % 2 of unit w / 2 of its four dim rows.
-  float vv[4][4];
-  auto fetch_v = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = kt + 4 * wv + i;
-      const float4 x = *(const float4*)(a.v_cache + (size_t)(key < k1 ? key : k0) * kHeadDim + 4 * lane);
-      vv[i][0] = key < k1 ? x.x : 0.f;
-      vv[i][1] = key < k1 ? x.y : 0.f;
-      vv[i][2] = key < k1 ? x.z : 0.f;
-      vv[i][3] = key < k1 ? x.w : 0.f;
-    }
-  };
-  auto stage_v = [&]() {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      bf16x4 hi, lo;
-      split4_bf16(vv[0][e], vv[1][e], vv[2][e], vv[3][e], hi, lo);
-      const int d = 4 * lane + e;
-      const int o = d * kPfKeys + 8 * ((wv >> 1) ^ ((d >> 1) & 3)) + 4 * (wv & 1);
-      *(bf16x4*)&Vh[o] = hi;
-      *(bf16x4*)&Vl[o] = lo;
-    }
-  };
-  fetch(a.k_cache, k0);
 
-  // q (normed + roped) of row l % 16, dims 32 t + 8 g .. +7, as bf16 hi / lo
-  const int row = qt * kPfRows + rt * 16 + c16;
-  const bool row_ok = row < M;
-  const int prow = a.pf_start + row, plo = pf_key_lo(a, prow);
-  const float sl2 = a.scale * 1.4426950408889634f;   // scores in log2 units (softmax in base 2)
-  // keys [kt, kt + 31] are valid for every row of the tile: all rows exist,
-  // the last key is <= the first row's position and < k1, and the first key
-  // is >= the last row's window start
-  const int r_first = a.pf_start + qt * kPfRows + rt * 16, r_last = r_first + 15;
-  const bool rows_full = qt * kPfRows + rt * 16 + 16 <= M;
-  const int lo_last = pf_key_lo(a, r_last);
-  auto tile_full = [&](int kt) { return rows_full && kt + kPfKeys - 1 <= r_first && kt + kPfKeys <= k1 && kt >= lo_last; };
-  const float* qp = a.qkv + (size_t)min(row, M - 1) * (nq * kHeadDim + 2 * kHeadDim) + min(h, nq - 1) * kHeadDim + 8 * g;
-  bf16x8 qh[8], ql[8];
+  int prow[2], plo[2];      // this lane's rows: position, first key
+  bool row_ok[2];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const float4 x0 = *(const float4*)(qp + 32 * t), x1 = *(const float4*)(qp + 32 * t + 4);
-    const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    uint32_t h4[4], l4[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) split2_bf16(xs[2 * e], xs[2 * e + 1], h4[e], l4[e]);
-    qh[t] = __builtin_bit_cast(bf16x8, h4);
-    ql[t] = __builtin_bit_cast(bf16x8, l4);
+  for (int rt = 0; rt < 2; ++rt) {
+    const int row = qt * kPfRows + 16 * rt + c16;
+    row_ok[rt] = row < M;
+    prow[rt] = a.pf_start + row;
+    plo[rt] = pf_key_lo(a, prow[rt]);
   }
-  stage_k();
+  // every key of the tile is valid for all 32 rows: all rows exist, the last
+  // key is at most the first row's position, the first key at least the last
+  // row's window start
+  const int r_first = a.pf_start + qt * kPfRows;
+  const bool rows_full = qt * kPfRows + kPfRows <= M;
+  const int lo_last = pf_key_lo(a, r_first + kPfRows - 1);
+  auto tile_full = [&](int t) {
+    return rows_full && t * kPfKeys + kPfKeys - 1 <= r_first && t * kPfKeys >= lo_last;
+  };
 
-  f32x4 o[16];
+  f32x4 o[2][16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
-  for (int kt = k0; kt < k1; kt += kPfKeys) {
-    fetch_v(kt);
-    __syncthreads();   // K of this tile staged; the previous tile's V reads done
-    float p[2][4];
-    float alpha = 1.f;
-    if (active) {
-      f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-      // S^T = K Q^T on bf16 MFMA: per 32 dims the products hi hi, lo hi and
-      // hi lo (the dropped lo lo term is below 2^-16 of |k| |q|). Operand row
-      // c16 of key tile j is key 8 (c16 / 4) + 4 j + c16 % 4, so register r of
-      // lane group g holds key 8 g + 4 j + r.
+  for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
+    for (int i = 0; i < 16; ++i) o[rt][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m[2] = {-INFINITY, -INFINITY}, mb[2] = {0.f, 0.f}, l[2] = {0.f, 0.f};
+  f32x4 s[2][2], nx[2][2];  // [row tile][key tile j]: scores of this and of the next tile
+  uint32_t ph[2][4], pl[2][4];
+
+  // The wave runs alone on its SIMD, so its instruction order is the schedule:
+  // it is written out and pinned slot by slot (fence), a few VALU instructions
+  // behind each pair of MFMAs, LDS operands read a whole group ahead.
+  auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+
+  // d[rt][j] = K Q^T of the K tile at kb: 8 dim blocks of 6 slots of two MFMAs
+  auto scores = [&](const uint8_t* kb, f32x4 (&d)[2][2], auto slot) __attribute__((always_inline)) {
+    bf16x8 k[2][4];
+    auto read = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int kr = 8 * (c16 >> 2) + 4 * j + (c16 & 3);
-          const int o = kr * kHeadDim + 8 * ((4 * t + g) ^ c16);
-          const bf16x8 kh = lds_bf16x8(&Kh[o]), kl = lds_bf16x8(&Kl[o]);
-          s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh[t], s[j], 0, 0, 0);
-          s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh[t], s[j], 0, 0, 0);
-          s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql[t], s[j], 0, 0, 0);
+      for (int x = 0; x < 4; ++x) k[t & 1][x] = lds_bf16x8(kb + (t * 4 + x) * 1024 + lane * 16);
+    };
+    read(0);
+    fence();
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      if (t < 7) read(t + 1);
+      fence();
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {   // (product, key tile); both row tiles
+        const int pr = q >> 1, j = q & 1;
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+          d[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[t & 1][2 * j + (pr == 1)], pr == 2 ? ql[rt][t] : qh[rt][t],
+                                                             t == 0 && pr == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[rt][j], 0, 0, 0);
+        slot(t * 6 + q);
+        fence();
+      }
+    }
+  };
+  // slot q of the softmax of tile t: probabilities 2 (q / 6) and + 1 of the
+  // lane's 16 are 2^(s - reference), added to the row's sum and split
+  float p0 = 0.f, p1 = 0.f, h0 = 0.f, h1 = 0.f;
+  auto probs = [&](int q) __attribute__((always_inline)) {
+    const int pair = q / 6, rt = pair >> 2, j = (pair >> 1) & 1, r = 2 * (pair & 1);
+    switch (q % 6) {
+      case 0:
+        p0 = s[rt][j][r] - mb[rt];
+        p1 = s[rt][j][r + 1] - mb[rt];
+        break;
+      case 1:
+        p0 = __builtin_amdgcn_exp2f(p0);
+        p1 = __builtin_amdgcn_exp2f(p1);
+        break;
+      case 2:
+        l[rt] += p0;
+        l[rt] += p1;
+        asm volatile("" : "+v"(l[rt]));
+        break;
+      case 3:
+        ph[rt][pair & 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){p0, p1}, bf16x2));
+        break;
+      case 4:
+        h0 = __uint_as_float(ph[rt][pair & 3] << 16);
+        h1 = __uint_as_float(ph[rt][pair & 3] & 0xffff0000u);
+        break;
+      case 5:
+        pl[rt][pair & 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){p0 - h0, p1 - h1}, bf16x2));
+        asm volatile("" : "+v"(pl[rt][pair & 3]));
+        break;
+    }
+    if (q % 6 < 2) asm volatile("" : "+v"(p0), "+v"(p1));   // or they sink past the MFMAs
+  };
+  // O += P V of the V tile at vb: 16 dim tiles of 3 slots of two MFMAs
+  auto weighted = [&](const uint8_t* vb, auto slot) __attribute__((always_inline)) {
+    bf16x8 v[3][2];
+    auto read = [&](int i) __attribute__((always_inline)) {
+      v[i % 3][0] = lds_bf16x8(vb + (i * 2) * 1024 + lane * 16);
+      v[i % 3][1] = lds_bf16x8(vb + (i * 2 + 1) * 1024 + lane * 16);
+    };
+    read(0);
+    read(1);
+    fence();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (i < 14) read(i + 2);
+      fence();
+#pragma unroll
+      for (int pr = 0; pr < 3; ++pr) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+          const u32x4 pf = pr == 1 ? u32x4{pl[rt][0], pl[rt][1], pl[rt][2], pl[rt][3]}
+                                   : u32x4{ph[rt][0], ph[rt][1], ph[rt][2], ph[rt][3]};
+          o[rt][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pf), v[i % 3][pr == 2], o[rt][i],
+                                                             0, 0, 0);
         }
+        slot(3 * i + pr);
+        fence();
       }
-      // scale (to log2 units) + causal / window mask; online softmax of row
-      // l % 16 in base 2. A tile inside every row's key range needs no mask.
-      float mx = -INFINITY;
-      if (tile_full(kt)) {
+    }
+  };
+  // causal / window mask of tile t's scores
+  auto mask = [&](int t, f32x4 (&d)[2][2]) __attribute__((always_inline)) {
+    if (tile_full(t)) return;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            p[j][r] = s[j][r] * sl2;
-            mx = fmaxf(mx, p[j][r]);
-          }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int key = kt + 8 * g + 4 * j + r;
-            const bool ok = row_ok && key < k1 && key >= plo && key <= prow;
-            p[j][r] = ok ? s[j][r] * sl2 : -INFINITY;
-            mx = fmaxf(mx, p[j][r]);
-          }
-      }
-      mx = pf_xor32_max(pf_xor16_max(mx));
-      const float mn = fmaxf(m, mx);
-      const float mb = mn == -INFINITY ? 0.f : mn;   // a row with no key yet keeps p = 0
-      alpha = __builtin_amdgcn_exp2f(m - mb);
-      float ps = 0.f;
+    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p[j][r] = __builtin_amdgcn_exp2f(p[j][r] - mb);
-          ps += p[j][r];
+          const int key = t * kPfKeys + 8 * g + 4 * j + r;
+          const bool ok = row_ok[rt] && key >= plo[rt] && key <= prow[rt];
+          d[rt][j][r] = ok ? d[rt][j][r] : -INFINITY;
         }
-      l = fmaf(l, alpha, ps);
-      m = mn;
-    }
-    __syncthreads();   // every K read of this tile done
-    stage_v();
-    if (kt + kPfKeys < k1) fetch(a.k_cache, kt + kPfKeys);
-    __syncthreads();   // V of this tile staged
-    if (active) {
-      // O rows 4 g + r take the factors of the lanes that hold those rows
-      // (skipped when no row's running max moved: every factor is then 1)
-      if (__ballot(alpha != 1.f)) {
+  };
+  // row maxima of the scores d, one of the lane's 16 per slot, then across
+  // the four lane groups
+  float mx[2];
+  auto maxima = [&](const f32x4 (&d)[2][2], int q) __attribute__((always_inline)) {
+    const int rt = (q >> 3) & 1;
+    if (q < 16) mx[rt] = (q & 7) == 0 ? d[rt][0][0] : fmaxf(mx[rt], d[rt][(q >> 2) & 1][q & 3]);
+    else if (q < 18) mx[q - 16] = pf_xor16_max(mx[q - 16]);
+    else if (q < 20) mx[q - 18] = pf_xor32_max(mx[q - 18]);
+  };
+  // moves the softmax reference where a row needs it
+  auto settle = [&]() __attribute__((always_inline)) {
+    const bool mv0 = mx[0] > m[0] + 8.f, mv1 = mx[1] > m[1] + 8.f;
+    if (__ballot(mv0 || mv1)) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const float mn = (rt ? mv1 : mv0) ? mx[rt] : m[rt];
+        const float nb = mn == -INFINITY ? 0.f : mn;   // a row with no key yet keeps p = 0
+        const float alpha = __builtin_amdgcn_exp2f(m[rt] - nb);
+        m[rt] = mn;
+        mb[rt] = nb;
+        l[rt] *= alpha;
+        // O rows 4 g + r take the factors of the lanes that hold those rows
         float ar[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g + r, 64);
 #pragma unroll
         for (int i = 0; i < 16; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[i][r] *= ar[r];
-      }
-      // O += P V on bf16 MFMA: A = P (row l % 16, keys 8 g .. 8 g + 7 =
-      // p[j][r] for key 8 g + 4 j + r), B = V^T rows; hi.hi, lo.hi, hi.lo
-      uint32_t ph4[4], pl4[4];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        split2_bf16(p[j][0], p[j][1], ph4[2 * j], pl4[2 * j]);
-        split2_bf16(p[j][2], p[j][3], ph4[2 * j + 1], pl4[2 * j + 1]);
-      }
-      const bf16x8 ph = __builtin_bit_cast(bf16x8, ph4), pl = __builtin_bit_cast(bf16x8, pl4);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int d = 16 * i + c16;
-        const int ov = d * kPfKeys + 8 * (g ^ ((d >> 1) & 3));
-        const bf16x8 vh = lds_bf16x8(&Vh[ov]), vl = lds_bf16x8(&Vl[ov]);
-        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vh, o[i], 0, 0, 0);
-        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vh, o[i], 0, 0, 0);
-        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vl, o[i], 0, 0, 0);
+          for (int r = 0; r < 4; ++r) o[rt][i][r] *= ar[r];
       }
     }
-    if (kt + kPfKeys < k1) stage_k();   // no K reads until the next barrier
+  };
+
+  arrived();
+  __syncthreads();
+  scores(Ks[0], s, [](int) {});
+  mask(tb, s);
+#pragma unroll
+  for (int q = 0; q < 20; ++q) maxima(s, q);
+  settle();
+  for (int t = tb; t + 1 < te; ++t) {
+    const int b = (t - tb) & 1;   // stage of V of tile t; K of tile t + 1 is in the other
+    // V stage b ^ 1 (tile t - 1) and K stage b (tile t) were last read before
+    // the previous barrier
+    copy(t + 1, 1, Vs[b ^ 1]);
+    copy(min(t + 2, te - 1), 0, Ks[b]);
+    scores(Ks[b ^ 1], nx, probs);
+    mask(t + 1, nx);
+    weighted(Vs[b], [&](int q) { maxima(nx, q); });
+    settle();
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) s[rt][j] = nx[rt][j];
+    arrived();
+    __syncthreads();
   }
-  if (!active) return;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  float lr[4], mr[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    lr[r] = __shfl(l, 4 * g + r, 64);
-    mr[r] = __shfl(m, 4 * g + r, 64);
-  }
+  for (int q = 0; q < 48; ++q) probs(q);
+  weighted(Vs[(te - 1 - tb) & 1], [](int) {});
+  if (h >= nq) return;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int orow = qt * kPfRows + rt * 16 + 4 * g + r;
-    if (orow >= M) continue;
-    if (nkc == 1) {
-      uint16_t* out = a.pf_out + ((size_t)orow * nq + h) * kHeadDim * 2;
-      const float il = 1.f / lr[r];
+  for (int rt = 0; rt < 2; ++rt) {
+    float lt = l[rt];
+    lt += __shfl_xor(lt, 16, 64);
+    lt += __shfl_xor(lt, 32, 64);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int e = a_slot(16 * i + c16);
-        split_bf16(o[i][r] * il, &out[e], &out[e + 32]);
-      }
-    } else {
-      float* pp = a.part + (((size_t)orow * kPrefillChunks + kc) * nq + h) * (2 + kHeadDim);
+    for (int r = 0; r < 4; ++r) {
+      const float lr = __shfl(lt, 4 * g + r, 64), mr = __shfl(m[rt], 4 * g + r, 64);
+      const int orow = qt * kPfRows + 16 * rt + 4 * g + r;
+      if (orow >= M) continue;
+      if (nkc == 1) {
+        uint16_t* out = a.pf_out + ((size_t)orow * nq + h) * kHeadDim * 2;
+        const float il = 1.f / lr;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) pp[2 + 16 * i + c16] = o[i][r];
-      if (c16 == 0) {
-        pp[0] = mr[r];
-        pp[1] = lr[r];
+        for (int i = 0; i < 16; i += 2) {   // dims 16 i + 2 c16 and + 1
+          uint32_t hi, lo;
+          split2_bf16(o[rt][i][r] * il, o[rt][i + 1][r] * il, hi, lo);
+          uint16_t* e = out + a_slot(16 * i + 2 * c16);
+          *(uint32_t*)e = hi;
+          *(uint32_t*)(e + 32) = lo;
+        }
+      } else {
+        float* pp = a.part + (((size_t)orow * kPrefillChunks + kc) * nq + h) * (2 + kHeadDim);
+#pragma unroll
+        for (int i = 0; i < 16; i += 2)
+          *(float2*)(pp + 2 + 16 * i + 2 * c16) = make_float2(o[rt][i][r], o[rt][i + 1][r]);
+        if (c16 == 0) {
+          pp[0] = mr;
+          pp[1] = lr;
+        }
       }
     }
   }
@@ -1197,8 +1244,8 @@ __global__ __launch_bounds__(256) void k_attn_pf_merge(AttnArgs a) {
   // (16-byte loads of each chunk's o); the same per-element sums, in chunk
   // order, as one thread per dim
   const int row = blockIdx.x, tid = threadIdx.x, nq = a.n_q, h = tid >> 6, d4 = tid & 63;
-  int klo, khi, nkc;
-  pf_tile_span(a, row / kPfRows, &klo, &khi, &nkc);
+  int t0, t1, nkc;
+  pf_tile_span(a, row / kPfRows, &t0, &t1, &nkc);
   if (nkc == 1 || h >= nq) return;
   const float* pr = a.part + (size_t)row * kPrefillChunks * nq * (2 + kHeadDim);
   // chunks in groups of four, each group's loads issued together (clamped
@@ -1593,62 +1640,140 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
   }
 }
 
-// One block per prompt row: RMSNorm + NEOX RoPE of the key head (into the
-// cache, with v) and of every query head, the latter in place in the QKV
-// rows for the attention kernel (fusedPerHeadNormRope, shaders.ts:420-467).
-__global__ __launch_bounds__(320) void k_rows_kv(RowArgs a) {
-  // wave w < n_q: query head w of the row, in place; wave n_q: the key head
-  // (into the cache) and the value row. Lane l holds dims l + 64 j, so the
-  // NEOX pairs (i, i + 128) are its own j and j + 2, and the head's sum of
-  // squares is one wave reduction: no LDS, no barrier
-  const int row = blockIdx.x, wv = threadIdx.x >> 6, lane = threadIdx.x & 63, nq = a.n_q;
-  if (wv > nq) return;
-  const int pos = a.pf_start + row;
-  float* qrow = const_cast<float*>(a.qkv) + (size_t)row * (nq * kHeadDim + 2 * kHeadDim);
-  float* src = qrow + wv * kHeadDim;   // wave nq: the key head
-  const float* w = wv < nq ? a.q_norm : a.k_norm;
-  const float* rt = a.rope + (size_t)pos * kHeadDim;
+// QK-norm + NEOX RoPE of every row's heads, k and v into the cache
+// (fusedPerHeadNormRope, shaders.ts:420-467), and q, k, v as bf16 hi / lo in
+// the attention kernel's MFMA operand order, each value split once. One block
+// per 8 aligned positions from the first key that this slice's attention
+// reads (kv_lo) to the end of its last 32-key tile: positions before the
+// slice are converted from the cache, positions past its end are zeros (a
+// masked key's probability 0 must meet a finite v). Wave w < n_q: query head
+// w; wave n_q: keys; wave n_q + 1: values. Lane l holds dims l + 64 j, so the
+// NEOX pairs (i, i + 128) are its own j and j + 2, and a head's sum of squares
+// is one wave reduction; the eight positions' loads are all in flight at
+// once. The operand order is reached through LDS in 16-byte units: a unit of
+// v holds eight keys of one dim, which is why a block takes eight positions.
+constexpr int kKvPos = 8;
+constexpr int kKvPitch = kHeadDim + 4;   // floats: eight rows' units fall into distinct banks
+__global__ __launch_bounds__(64 * (kAttnMaxQ + 2)) void k_rows_kv(RowArgs a) {
+  __shared__ __align__(16) float xs[kKvPos * (kAttnMaxQ + 2) * kKvPitch];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, nq = a.n_q, nh = nq + 2;
+  const int p0 = (a.kv_lo / kPfKeys) * kPfKeys + kKvPos * blockIdx.x;
+  const int row0 = p0 - a.pf_start;
+  const bool is_q = wv < nq, is_v = wv == nq + 1;
+  const size_t stride = (size_t)nh * kHeadDim;
+  auto fresh = [&](int i) { return row0 + i >= 0 && row0 + i < a.M; };
+  float x[kKvPos][4];
+  // every load is issued unconditionally (rows clamped into the slice, cache
+  // rows into the context read so far) so that all of them are in flight together
+  auto row_of = [&](int i) { return min(max(row0 + i, 0), a.M - 1); };
+#pragma unroll
+  for (int i = 0; i < kKvPos; ++i) {
+    const float* src = a.qkv + (size_t)row_of(i) * stride + wv * kHeadDim;
+    if (!is_q && row0 + i < 0) src = (is_v ? a.v_cache : a.k_cache) + (size_t)(p0 + i) * kHeadDim;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[i][j] = src[lane + 64 * j];
+  }
   // the QKV GEMM's K slices (pre_planes of them, pre_stride floats apart)
-  // are added in slice order; the sum stays in slice 0
-  const int ns = a.pre_planes > 1 ? a.pre_planes : 1;
-  float x[4], nw[4], cs[2], sn[2];
+  // are added in slice order
+  float y[kQkvMaxSlices - 1][kKvPos][4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    x[j] = src[lane + 64 * j];
-    nw[j] = w[lane + 64 * j];
+  for (int p = 1; p < kQkvMaxSlices; ++p)
+    if (p < a.pre_planes)
+#pragma unroll
+      for (int i = 0; i < kKvPos; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          y[p - 1][i][j] = a.qkv[p * a.pre_stride + (size_t)row_of(i) * stride + wv * kHeadDim + lane + 64 * j];
+#pragma unroll
+  for (int p = 1; p < kQkvMaxSlices; ++p)
+    if (p < a.pre_planes)
+#pragma unroll
+      for (int i = 0; i < kKvPos; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[i][j] += fresh(i) ? y[p - 1][i][j] : 0.f;
+  if (!is_v && row0 + kKvPos > 0) {
+    const float* w = is_q ? a.q_norm : a.k_norm;
+    float nw[4], cs[kKvPos][2], sn[kKvPos][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) nw[j] = w[lane + 64 * j];
+#pragma unroll
+    for (int i = 0; i < kKvPos; ++i) {
+      const float* rt = a.rope + (size_t)(a.pf_start + row_of(i)) * kHeadDim;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        cs[i][j] = rt[lane + 64 * j];
+        sn[i][j] = rt[kHeadDim / 2 + lane + 64 * j];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kKvPos; ++i) {
+      float ss = 0.f, y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss = fmaf(x[i][j], x[i][j], ss);
+      const float ri = rsq(wave_sum_dpp(ss) / (float)kHeadDim + a.eps);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = (x[i][j] * nw[j]) * ri;
+      if (fresh(i))
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          x[i][j] = y[j] * cs[i][j] - y[j + 2] * sn[i][j];
+          x[i][j + 2] = y[j] * sn[i][j] + y[j + 2] * cs[i][j];
+        }
+    }
   }
-  for (int p = 1; p < ns; ++p)
+  if (!is_q) {
+    float* cache = is_v ? a.v_cache : a.k_cache;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x[j] += src[p * a.pre_stride + lane + 64 * j];
+    for (int i = 0; i < kKvPos; ++i)
+      if (fresh(i))
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    cs[j] = rt[lane + 64 * j];
-    sn[j] = rt[kHeadDim / 2 + lane + 64 * j];
+        for (int j = 0; j < 4; ++j) cache[(size_t)(p0 + i) * kHeadDim + lane + 64 * j] = x[i][j];
   }
-  float v[4];
-  if (wv == nq) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = src[kHeadDim + lane + 64 * j];
-    for (int p = 1; p < ns; ++p)
+  for (int i = 0; i < kKvPos; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] += src[p * a.pre_stride + kHeadDim + lane + 64 * j];
+    for (int j = 0; j < 4; ++j)   // positions past the slice: zeros
+      xs[(i * nh + wv) * kKvPitch + lane + 64 * j] = row0 + i < a.M ? x[i][j] : 0.f;
+  __syncthreads();
+
+  const int tid = threadIdx.x, nt = 64 * nh;
+  auto split8 = [](const float* v, uint16_t* hi, uint16_t* lo) {
+    uint32_t h4[4], l4[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split2_bf16(v[2 * e], v[2 * e + 1], h4[e], l4[e]);
+    *(u32x4*)hi = u32x4{h4[0], h4[1], h4[2], h4[3]};
+    *(u32x4*)lo = u32x4{l4[0], l4[1], l4[2], l4[3]};
+  };
+  uint16_t* tile = (uint16_t*)(a.kv_planes + (size_t)(p0 / kPfKeys) * kKvTileBytes);
+  // heads 0 .. n_q - 1 (q, scaled) and n_q (k): unit = (position, 8 dims)
+  for (int u = tid; u < (nq + 1) * 256; u += nt) {
+    const int i = u & 7, c = (u >> 3) & 31, hd = u >> 8, t = c >> 2, gd = c & 3;
+    float v[8];
+    const float4* src = (const float4*)&xs[(i * nh + hd) * kKvPitch + 8 * c];
+    const float4 v0 = src[0], v1 = src[1];
+    v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
+    v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
+    uint16_t* dst;
+    if (hd < nq) {
+      const int row = row0 + i;
+      if (row < 0 || row >= a.M) continue;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= a.q_scale;
+      dst = a.q_frag + ((size_t)((row >> 4) * nq + hd) * 16 + 2 * t) * 512 + (gd * 16 + (row & 15)) * 8;
+    } else {
+      const int kk = (p0 + i) % kPfKeys, j = (kk >> 2) & 1, r = (kk >> 3) * 4 + (kk & 3);
+      dst = tile + ((t * 2 + j) * 2) * 512 + (gd * 16 + r) * 8;
+    }
+    split8(v, dst, dst + 512);
   }
-  float ss = 0.f;
+  // v: unit = (dim, this block's eight keys)
+  for (int d = tid; d < kHeadDim; d += nt) {
+    float v[8];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) ss = fmaf(x[j], x[j], ss);
-  const float ri = rsq(wave_sum_dpp(ss) / (float)kHeadDim + a.eps);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) x[j] = (x[j] * nw[j]) * ri;
-  float* dst = wv < nq ? src : a.k_cache + (size_t)pos * kHeadDim;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const float x0 = x[j], x1 = x[j + 2];
-    dst[lane + 64 * j] = x0 * cs[j] - x1 * sn[j];
-    dst[lane + 64 * j + 128] = x0 * sn[j] + x1 * cs[j];
-  }
-  if (wv == nq) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a.v_cache[(size_t)pos * kHeadDim + lane + 64 * j] = v[j];
+    for (int i = 0; i < kKvPos; ++i) v[i] = xs[(i * nh + nq + 1) * kKvPitch + d];
+    const int dt = 2 * (d >> 5) + (d & 1), c = (d & 31) >> 1;   // dim tile and column: adjacent dims in one lane
+    uint16_t* dst = tile + kPfTile / 2 + (dt * 2) * 512 + (((p0 % kPfKeys) / kKvPos) * 16 + c) * 8;
+    split8(v, dst, dst + 512);
   }
 }
 
@@ -1946,13 +2071,12 @@ int launch_attention_merge(const AttnArgs& a, int chunks, void* stream) {
 }
 
 int launch_prefill_attention(const AttnArgs& a, int M, void* stream) {
-  if (a.n_q < 1 || a.n_q > kAttnMaxQ || M < 1 || a.pf_rows != M || a.pf_start < 0 || a.window < 0 ||
-      a.pf_chunk < kPfKeys || a.pf_chunk % kPfKeys)
+  if (a.n_q < 1 || a.n_q > kAttnMaxQ || M < 1 || a.pf_rows != M || a.pf_start < 0 || a.window < 0 || a.pf_chunk < 1 ||
+      !a.q_frag || !a.kv_planes)
     return (int)hipErrorInvalidValue;
-  const int span = prefill_max_span(a.window, a.pf_start, M);
-  const int nkc = (span + a.pf_chunk - 1) / a.pf_chunk;
+  const int nkc = (prefill_max_tiles(a.window, a.pf_start, M) + a.pf_chunk - 1) / a.pf_chunk;
   if (nkc > kPrefillChunks) return (int)hipErrorInvalidValue;   // `part` holds kPrefillChunks per row
-  hipLaunchKernelGGL(k_attn_pf, dim3(nkc, (M + kPfRows - 1) / kPfRows), dim3(512), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(k_attn_pf, dim3(nkc, (M + kPfRows - 1) / kPfRows), dim3(256), 0, (hipStream_t)stream, a);
   if (nkc > 1) hipLaunchKernelGGL(k_attn_pf_merge, dim3(M), dim3(256), 0, (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
@@ -2077,11 +2201,13 @@ int launch_rows_resid(const RowArgs& a, void* stream) {
 }
 
 int launch_rows_kv(const RowArgs& a, void* stream) {
-  if (a.M < 1) return (int)hipErrorInvalidValue;
-  if (a.n_q < 1 || a.n_q > kAttnMaxQ || a.pre_planes > kGemmMaxSlices ||
+  if (a.M < 1 || a.kv_lo < 0 || a.kv_lo > a.pf_start || !a.q_frag || !a.kv_planes) return (int)hipErrorInvalidValue;
+  if (a.n_q < 1 || a.n_q > kAttnMaxQ || a.pre_planes > kQkvMaxSlices ||
       (a.pre_planes > 1 && a.pre_stride < (size_t)a.M * (a.n_q + 2) * kHeadDim))
     return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_rows_kv, dim3(a.M), dim3(64 * (a.n_q + 1)), 0, (hipStream_t)stream, a);
+  const int first = a.kv_lo / kPfKeys, last = (a.pf_start + a.M - 1) / kPfKeys;
+  hipLaunchKernelGGL(k_rows_kv, dim3((last - first + 1) * (kPfKeys / kKvPos)), dim3(64 * (a.n_q + 2)), 0,
+                     (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
 

@@ -121,6 +121,9 @@ struct gg_ctx {
   float *pf_hidden = nullptr, *pf_residual = nullptr, *pf_qkv = nullptr, *pf_o = nullptr, *pf_part = nullptr;
   // GEMM inputs as bf16 hi / lo (the slice's M rows each)
   uint16_t *pf_xn = nullptr, *pf_attn = nullptr, *pf_act = nullptr;
+  // attention operands of the current layer: q of the slice, k / v of the context
+  uint16_t* pf_qfrag = nullptr;
+  uint8_t* pf_planes = nullptr;
 
   // pinned host mirrors
   DevState* h_st = nullptr;
@@ -642,8 +645,9 @@ int sync(gg_ctx* c, const char* what) {
 // that minimise the modelled time: the 32-wide steps of a block times the
 // fitted time of a step with as many blocks on the CU as this launch puts
 // there (kGemmTiles; 0.3 of the round-up to whole blocks per CU counts, the
-// rest overlaps), plus 8 bytes per output of each slice at 5 TB/s for writing
-// it and for the consumer's read. Over the timings that the fit used, the
+// rest overlaps), plus 6 bytes per output of each slice at 5 TB/s for writing
+// it and for the consumer's read (down at 2048 rows: 81 us and 11.5 us in the
+// row kernel with two slices, 70 and 14 us with four). Over the timings that the fit used, the
 // choice is 4% slower than the best tile and split on average and 21% at
 // worst, while the best fixed tile of a matrix is off by 2x at the ends.
 void gemm_plan(GemmArgs& g, int max_ks, bool out) {
@@ -659,7 +663,7 @@ void gemm_plan(GemmArgs& g, int max_ks, bool out) {
       const double blocks = (double)tiles * ks;
       const double per_cu = 0.7 * std::max(1.0, blocks / 256) + 0.3 * std::ceil(blocks / 256);
       const double cost = (steps / ks) * (T.lat + T.thr * (per_cu - 1.0)) +
-                          (out ? ks * ((double)g.M * g.N * 8 / 5e6) : 0.0);
+                          (out ? ks * ((double)g.M * g.N * 6 / 5e6) : 0.0);
       if (g.tile < 0 || cost < best) {
         best = cost;
         g.tile = t;
@@ -721,14 +725,17 @@ int prefill_slice(gg_ctx* c, const int32_t* d_tokens, int M, int start) {
     kv.rope = swa ? c->rope_local : c->rope_global;
     kv.k_cache = Ly.kc;
     kv.v_cache = Ly.vc;
+    const int window = swa ? c->c.sliding_window : 0;
+    kv.kv_lo = window > 0 ? std::max(0, start - window + 1) : 0;
+    kv.q_scale = (float)(1.4426950408889634 / std::sqrt((double)kHeadDim));
+    kv.q_frag = c->pf_qfrag;
+    kv.kv_planes = c->pf_planes;
     GG_TRY(launch_rc(c, launch_rows_kv(kv, s), "prefill kv"));
     AttnArgs at{};
-    at.qkv = c->pf_qkv;
     at.n_q = c->NQ;
-    at.k_cache = Ly.kc;
-    at.v_cache = Ly.vc;
-    at.window = swa ? c->c.sliding_window : 0;
-    at.scale = (float)(1.0 / std::sqrt((double)kHeadDim));
+    at.window = window;
+    at.q_frag = c->pf_qfrag;
+    at.kv_planes = c->pf_planes;
     at.part = c->pf_part;
     at.pf_out = c->pf_attn;
     at.pf_start = start;
@@ -1058,6 +1065,8 @@ int gg_finalize(gg_ctx* c) {
     GG_TRY(dalloc(c, &c->pf_qkv, (size_t)std::max(qkv_slices(M) * M, qkv_slices(few) * few) * c->NQKV * 4));
     GG_TRY(dalloc(c, &c->pf_attn, (size_t)M * c->QD * 4));
     GG_TRY(dalloc(c, &c->pf_act, (size_t)M * c->I * 4));
+    GG_TRY(dalloc(c, &c->pf_qfrag, (size_t)cdiv(M, 32) * 32 * c->QD * 4));
+    GG_TRY(dalloc(c, &c->pf_planes, (size_t)cdiv(c->CTX, 32) * kKvTileBytes));
     GG_TRY(dalloc(c, &c->pf_part, (size_t)M * kPrefillChunks * kAttnMaxQ * (2 + kHeadDim) * 4));
   }
   GG_HIP(c, hipMemset(c->seen, 0, (size_t)cdiv(c->V, 32) * 4));
