@@ -1557,24 +1557,31 @@ __global__ __launch_bounds__(256) void k_rows_embed(RowArgs a) {
   row_norm_out(h, a.w_pre, H, a.eps, a.x_out + (size_t)row * H * 2, sh4, n);
 }
 
+// One block per prompt row: thread t holds float4s t and t + 256, so every
+// load of the row (all K slices of the GEMM output, the residual, both norm
+// weights) is in flight before the sums. Memory-bound at thousands of rows
+// (4096 rows, two slices, 94 MB: 19.1 -> 16.9 us), one memory latency and two
+// barriers at few: 187 rows 8.6 -> 4.6 us, 64 rows of 640 6.1 -> 3.5 us,
+// against one wave per row.
 __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
-  // one wave per prompt row, four rows per block: lane l holds float4s
-  // l + 64 k of the row, so both sums of squares are wave reductions (no
-  // LDS, no barrier); every load of the row is issued before the sums
-  constexpr int KF = 2048 / 4 / 64;   // float4s per lane at the largest hidden size
-  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), H = a.H;
-  if (row >= a.M) return;
+  constexpr int KF = 2048 / 4 / 256;   // float4s per thread at the largest hidden size
+  __shared__ float sh[2][4];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, H = a.H, row = blockIdx.x;
   const int F4 = H / 4;
   const size_t o4 = (size_t)row * F4;
   const float4* pre = (const float4*)a.pre;
   const float4* res = (const float4*)a.res;
-  const float4* wpost = (const float4*)a.w_post;
-  const float4* wpre = (const float4*)a.w_pre;
   const size_t ps4 = a.pre_stride / 4;
-  float4 v[KF], rs[KF], wq[KF];
+  auto sum_row = [&](float x, int i) {
+    x = wave_sum_dpp(x);
+    if (lane == 0) sh[i][wv] = x;
+    __syncthreads();
+    return (sh[i][0] + sh[i][1]) + (sh[i][2] + sh[i][3]);
+  };
+  float4 v[KF], rs[KF], wq[KF], wp[KF];
 #pragma unroll
   for (int k = 0; k < KF; ++k) {
-    const int f = lane + 64 * k;
+    const int f = tid + 256 * k;
     if (f < F4) {
       v[k] = pre[o4 + f];
       float4 pv[kGemmMaxSlices - 1];
@@ -1582,7 +1589,8 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
       for (int p = 1; p < kGemmMaxSlices; ++p)
         if (p < a.pre_planes) pv[p - 1] = pre[p * ps4 + o4 + f];
       rs[k] = res[o4 + f];
-      wq[k] = wpost[f];
+      wq[k] = ((const float4*)a.w_post)[f];
+      wp[k] = ((const float4*)a.w_pre)[f];
       // K slices of the previous GEMM, added in slice order
 #pragma unroll
       for (int p = 1; p < kGemmMaxSlices; ++p)
@@ -1597,17 +1605,17 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
   float s1 = 0.f;
 #pragma unroll
   for (int k = 0; k < KF; ++k)
-    if (lane + 64 * k < F4) {
+    if (tid + 256 * k < F4) {
       s1 = fmaf(v[k].x, v[k].x, s1);
       s1 = fmaf(v[k].y, v[k].y, s1);
       s1 = fmaf(v[k].z, v[k].z, s1);
       s1 = fmaf(v[k].w, v[k].w, s1);
     }
-  const float ri1 = rsq(wave_sum_dpp(s1) / (float)H + a.eps);
+  const float ri1 = rsq(sum_row(s1, 0) / (float)H + a.eps);
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < KF; ++k) {
-    const int f = lane + 64 * k;
+    const int f = tid + 256 * k;
     if (f < F4) {
       float4 r;
       r.x = rs[k].x + (v[k].x * wq[k].x) * ri1;
@@ -1623,19 +1631,17 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
       ss = fmaf(r.w, r.w, ss);
     }
   }
-  const float ri = rsq(wave_sum_dpp(ss) / (float)H + a.eps);
+  const float ri = rsq(sum_row(ss, 1) / (float)H + a.eps);
 #pragma unroll
   for (int k = 0; k < KF; ++k) {
-    const int f = lane + 64 * k;
+    const int f = tid + 256 * k;
     if (f < F4) {
-      const float4 w = wpre[f];
-      const float y[4] = {(v[k].x * w.x) * ri, (v[k].y * w.y) * ri, (v[k].z * w.z) * ri, (v[k].w * w.w) * ri};
-      uint16_t hi[4], lo[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) split_bf16(y[j], &hi[j], &lo[j]);
+      const float4 w = wp[k];
+      bf16x4 hi, lo;
+      split4_bf16((v[k].x * w.x) * ri, (v[k].y * w.y) * ri, (v[k].z * w.z) * ri, (v[k].w * w.w) * ri, hi, lo);
       uint16_t* xo = a.x_out + (size_t)row * H * 2 + a_slot(4 * f);
-      *(uint2*)xo = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-      *(uint2*)(xo + 32) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
+      *(bf16x4*)xo = hi;
+      *(bf16x4*)(xo + 32) = lo;
     }
   }
 }
@@ -1646,41 +1652,42 @@ __global__ __launch_bounds__(256) void k_rows_resid(RowArgs a) {
 // per 8 aligned positions from the first key that this slice's attention
 // reads (kv_lo) to the end of its last 32-key tile: positions before the
 // slice are converted from the cache, positions past its end are zeros (a
-// masked key's probability 0 must meet a finite v). Wave w < n_q: query head
-// w; wave n_q: keys; wave n_q + 1: values. Lane l holds dims l + 64 j, so the
+// masked key's probability 0 must meet a finite v). Waves w and w + n_q + 2 take
+// positions 0-3 and 4-7 of query head w, of the keys (w = n_q) or the values
+// (n_q + 1). Lane l holds dims l + 64 j, so the
 // NEOX pairs (i, i + 128) are its own j and j + 2, and a head's sum of squares
-// is one wave reduction; the eight positions' loads are all in flight at
-// once. The operand order is reached through LDS in 16-byte units: a unit of
+// is one wave reduction; a wave's loads are all in flight at once. The operand order is reached through LDS in 16-byte units: a unit of
 // v holds eight keys of one dim, which is why a block takes eight positions.
-constexpr int kKvPos = 8;
+constexpr int kKvPos = 8, kKvWavePos = 4;
 constexpr int kKvPitch = kHeadDim + 4;   // floats: eight rows' units fall into distinct banks
-__global__ __launch_bounds__(64 * (kAttnMaxQ + 2)) void k_rows_kv(RowArgs a) {
+__global__ __launch_bounds__(128 * (kAttnMaxQ + 2)) void k_rows_kv(RowArgs a) {
   __shared__ __align__(16) float xs[kKvPos * (kAttnMaxQ + 2) * kKvPitch];
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, nq = a.n_q, nh = nq + 2;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, nq = a.n_q, nh = nq + 2;
+  const int wv = wid >= nh ? wid - nh : wid, half = wid >= nh ? kKvWavePos : 0;
   const int p0 = (a.kv_lo / kPfKeys) * kPfKeys + kKvPos * blockIdx.x;
-  const int row0 = p0 - a.pf_start;
+  const int row0 = p0 - a.pf_start;   // the block's positions as rows; wave position i is half + i
   const bool is_q = wv < nq, is_v = wv == nq + 1;
   const size_t stride = (size_t)nh * kHeadDim;
-  auto fresh = [&](int i) { return row0 + i >= 0 && row0 + i < a.M; };
-  float x[kKvPos][4];
+  auto fresh = [&](int i) { return row0 + half + i >= 0 && row0 + half + i < a.M; };
+  float x[kKvWavePos][4];
   // every load is issued unconditionally (rows clamped into the slice, cache
   // rows into the context read so far) so that all of them are in flight together
-  auto row_of = [&](int i) { return min(max(row0 + i, 0), a.M - 1); };
+  auto row_of = [&](int i) { return min(max(row0 + half + i, 0), a.M - 1); };
 #pragma unroll
-  for (int i = 0; i < kKvPos; ++i) {
+  for (int i = 0; i < kKvWavePos; ++i) {
     const float* src = a.qkv + (size_t)row_of(i) * stride + wv * kHeadDim;
-    if (!is_q && row0 + i < 0) src = (is_v ? a.v_cache : a.k_cache) + (size_t)(p0 + i) * kHeadDim;
+    if (!is_q && row0 + half + i < 0) src = (is_v ? a.v_cache : a.k_cache) + (size_t)(p0 + half + i) * kHeadDim;
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[i][j] = src[lane + 64 * j];
   }
   // the QKV GEMM's K slices (pre_planes of them, pre_stride floats apart)
   // are added in slice order
-  float y[kQkvMaxSlices - 1][kKvPos][4];
+  float y[kQkvMaxSlices - 1][kKvWavePos][4];
 #pragma unroll
   for (int p = 1; p < kQkvMaxSlices; ++p)
     if (p < a.pre_planes)
 #pragma unroll
-      for (int i = 0; i < kKvPos; ++i)
+      for (int i = 0; i < kKvWavePos; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           y[p - 1][i][j] = a.qkv[p * a.pre_stride + (size_t)row_of(i) * stride + wv * kHeadDim + lane + 64 * j];
@@ -1688,16 +1695,16 @@ __global__ __launch_bounds__(64 * (kAttnMaxQ + 2)) void k_rows_kv(RowArgs a) {
   for (int p = 1; p < kQkvMaxSlices; ++p)
     if (p < a.pre_planes)
 #pragma unroll
-      for (int i = 0; i < kKvPos; ++i)
+      for (int i = 0; i < kKvWavePos; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) x[i][j] += fresh(i) ? y[p - 1][i][j] : 0.f;
-  if (!is_v && row0 + kKvPos > 0) {
+  if (!is_v && row0 + half + kKvWavePos > 0) {
     const float* w = is_q ? a.q_norm : a.k_norm;
-    float nw[4], cs[kKvPos][2], sn[kKvPos][2];
+    float nw[4], cs[kKvWavePos][2], sn[kKvWavePos][2];
 #pragma unroll
     for (int j = 0; j < 4; ++j) nw[j] = w[lane + 64 * j];
 #pragma unroll
-    for (int i = 0; i < kKvPos; ++i) {
+    for (int i = 0; i < kKvWavePos; ++i) {
       const float* rt = a.rope + (size_t)(a.pf_start + row_of(i)) * kHeadDim;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -1706,7 +1713,7 @@ __global__ __launch_bounds__(64 * (kAttnMaxQ + 2)) void k_rows_kv(RowArgs a) {
       }
     }
 #pragma unroll
-    for (int i = 0; i < kKvPos; ++i) {
+    for (int i = 0; i < kKvWavePos; ++i) {
       float ss = 0.f, y[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) ss = fmaf(x[i][j], x[i][j], ss);
@@ -1724,19 +1731,19 @@ __global__ __launch_bounds__(64 * (kAttnMaxQ + 2)) void k_rows_kv(RowArgs a) {
   if (!is_q) {
     float* cache = is_v ? a.v_cache : a.k_cache;
 #pragma unroll
-    for (int i = 0; i < kKvPos; ++i)
+    for (int i = 0; i < kKvWavePos; ++i)
       if (fresh(i))
 #pragma unroll
-        for (int j = 0; j < 4; ++j) cache[(size_t)(p0 + i) * kHeadDim + lane + 64 * j] = x[i][j];
+        for (int j = 0; j < 4; ++j) cache[(size_t)(p0 + half + i) * kHeadDim + lane + 64 * j] = x[i][j];
   }
 #pragma unroll
-  for (int i = 0; i < kKvPos; ++i)
+  for (int i = 0; i < kKvWavePos; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)   // positions past the slice: zeros
-      xs[(i * nh + wv) * kKvPitch + lane + 64 * j] = row0 + i < a.M ? x[i][j] : 0.f;
+      xs[((half + i) * nh + wv) * kKvPitch + lane + 64 * j] = row0 + half + i < a.M ? x[i][j] : 0.f;
   __syncthreads();
 
-  const int tid = threadIdx.x, nt = 64 * nh;
+  const int tid = threadIdx.x, nt = 128 * nh;
   auto split8 = [](const float* v, uint16_t* hi, uint16_t* lo) {
     uint32_t h4[4], l4[4];
 #pragma unroll
@@ -2196,7 +2203,7 @@ int launch_rows_embed(const RowArgs& a, void* stream) {
 int launch_rows_resid(const RowArgs& a, void* stream) {
   if (a.H > 2048 || a.M < 1) return (int)hipErrorInvalidValue;
   if (a.H % 4 || a.pre_stride % 4) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_rows_resid, dim3((a.M + 3) / 4), dim3(256), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(k_rows_resid, dim3(a.M), dim3(256), 0, (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
 
@@ -2206,7 +2213,7 @@ int launch_rows_kv(const RowArgs& a, void* stream) {
       (a.pre_planes > 1 && a.pre_stride < (size_t)a.M * (a.n_q + 2) * kHeadDim))
     return (int)hipErrorInvalidValue;
   const int first = a.kv_lo / kPfKeys, last = (a.pf_start + a.M - 1) / kPfKeys;
-  hipLaunchKernelGGL(k_rows_kv, dim3((last - first + 1) * (kPfKeys / kKvPos)), dim3(64 * (a.n_q + 2)), 0,
+  hipLaunchKernelGGL(k_rows_kv, dim3((last - first + 1) * (kPfKeys / kKvPos)), dim3(128 * (a.n_q + 2)), 0,
                      (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
