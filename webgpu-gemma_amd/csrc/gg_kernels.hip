@@ -1913,6 +1913,40 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t* __restrict__ src
   out[i] = (float)(int8_t)blk[2 + (i & 31)] * scale;
 }
 
+// The same for 16-byte aligned src and out: a block takes 128 Q8_0 blocks
+// (4352 bytes, a multiple of 16) through LDS in 16-byte loads and writes 4096
+// floats in 16-byte stores; the byte loads and 4-byte stores above keep a
+// quarter of the bytes in flight (8 M values, 40 MB: 12.4 -> 7.9 us).
+constexpr int kDeqBlocks = 128;
+__global__ __launch_bounds__(256) void k_dequant16(const uint8_t* __restrict__ src, float* __restrict__ out,
+                                                   long long nblk) {
+  __shared__ __align__(16) uint8_t s[kDeqBlocks * 34];
+  const int tid = threadIdx.x;
+  const long long b0 = (long long)blockIdx.x * kDeqBlocks;
+  const int nb = (int)(nblk - b0 < kDeqBlocks ? nblk - b0 : kDeqBlocks);
+  const int bytes = nb * 34;
+  const uint8_t* p = src + b0 * 34;
+  for (int u = tid; u < kDeqBlocks * 34 / 16; u += 256) {
+    if (16 * u + 16 <= bytes) *(u32x4*)&s[16 * u] = ((const u32x4*)p)[u];
+    else
+      for (int e = 16 * u; e < bytes; ++e) s[e] = p[e];   // the last block's tail
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = tid + 256 * j, q = i >> 3;   // float4 i: block q, values 4 (i % 8) .. + 3
+    if (q < nb) {
+      const uint16_t* h = (const uint16_t*)&s[q * 34];
+      const float scale = (float)__builtin_bit_cast(_Float16, h[0]);
+      const uint32_t w = h[1 + 2 * (i & 7)] | ((uint32_t)h[2 + 2 * (i & 7)] << 16);
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (float)(int8_t)(w >> (8 * e)) * scale;
+      *((f32x4*)(out + b0 * 32) + i) = o;
+    }
+  }
+}
+
 // GGUF Q8_0 rows -> the prefill GEMM's weights: int8 values as bf16 (exact)
 // and fp32 block scales, one thread per 32-block. Source row r goes to row
 // r + off, or with half = 16 to (r / 16) * 32 + r % 16 + off (gate / up
@@ -2155,6 +2189,12 @@ int launch_q8_bf16(const uint8_t* src, uint16_t* wb, float* wd, long long rows, 
 
 int launch_dequant(const uint8_t* src, float* out, long long n, void* stream) {
   if (n <= 0) return 0;
+  if (n % 32 == 0 && ((uintptr_t)src | (uintptr_t)out) % 16 == 0) {
+    const long long nblk = n / 32;
+    hipLaunchKernelGGL(k_dequant16, dim3((unsigned)((nblk + kDeqBlocks - 1) / kDeqBlocks)), dim3(256), 0,
+                       (hipStream_t)stream, src, out, nblk);
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(k_dequant, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, src, out,
                      n);
   return (int)hipGetLastError();
