@@ -1968,10 +1968,16 @@ __global__ __launch_bounds__(256) void k_q8_bf16(const uint8_t* __restrict__ src
   const int r16 = (int)(R & 15);
   wd[tb * 16 + r16] = (float)__builtin_bit_cast(_Float16, (uint16_t)(blk[0] | (blk[1] << 8)));
 #pragma unroll
-  for (int f = 0; f < 32; ++f) {
-    const int p = act_order ? act_slot(f) : f;
-    wb[tb * 512 + ((p >> 3) * 16 + r16) * 8 + (p & 7)] =
-        (uint16_t)(__float_as_uint((float)(int8_t)blk[2 + f]) >> 16);
+  for (int g = 0; g < 4; ++g) {   // operand slots 8 g .. + 7
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int p = 8 * g + 2 * e;   // slots p, p + 1 hold inputs p, p + 1 or (act_slot) p / 2, p / 2 + 16
+      const float f0 = (float)(int8_t)blk[2 + (act_order ? p / 2 : p)];
+      const float f1 = (float)(int8_t)blk[2 + (act_order ? p / 2 + 16 : p + 1)];
+      o[e] = (__float_as_uint(f0) >> 16) | (__float_as_uint(f1) & 0xffff0000u);
+    }
+    *(u32x4*)(wb + tb * 512 + (g * 16 + r16) * 8) = u32x4{o[0], o[1], o[2], o[3]};
   }
 }
 
