@@ -1947,6 +1947,19 @@ __global__ __launch_bounds__(256) void k_dequant16(const uint8_t* __restrict__ s
   }
 }
 
+// Class-major logits (row c + 256 k at c * V / 256 + k, as the persistent
+// decode kernel leaves them) back in row order: 64 x 64 tiles through LDS.
+__global__ __launch_bounds__(256) void k_logits_rows(const float* __restrict__ cm, float* __restrict__ out, int R) {
+  __shared__ float t[64][65];
+  const int x = threadIdx.x & 63, y0 = threadIdx.x >> 6;
+  const int k0 = 64 * blockIdx.x, c0 = 64 * blockIdx.y;
+  for (int y = y0; y < 64; y += 4)
+    if (k0 + x < R) t[y][x] = cm[(size_t)(c0 + y) * R + k0 + x];
+  __syncthreads();
+  for (int y = y0; y < 64; y += 4)
+    if (k0 + y < R) out[(size_t)(k0 + y) * 256 + c0 + x] = t[x][y];
+}
+
 // GGUF Q8_0 rows -> the prefill GEMM's weights: int8 values as bf16 (exact)
 // and fp32 block scales, one thread per 32-block. Source row r goes to row
 // r + off, or with half = 16 to (r / 16) * 32 + r % 16 + off (gate / up
@@ -2190,6 +2203,13 @@ int launch_q8_bf16(const uint8_t* src, uint16_t* wb, float* wd, long long rows, 
   if (total <= 0) return 0;
   hipLaunchKernelGGL(k_q8_bf16, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, src, wb,
                      wd, rows, K, off, half, act_order);
+  return (int)hipGetLastError();
+}
+
+int launch_logits_rows(const float* cm, float* out, int V, void* stream) {
+  if (V <= 0 || V % 256) return (int)hipErrorInvalidValue;
+  const int R = V / 256;
+  hipLaunchKernelGGL(k_logits_rows, dim3((R + 63) / 64, 4), dim3(256), 0, (hipStream_t)stream, cm, out, R);
   return (int)hipGetLastError();
 }
 

@@ -107,6 +107,7 @@ struct gg_ctx {
   float *act = nullptr, *down_out = nullptr, *hidden = nullptr, *residual = nullptr, *normed = nullptr;
   float *logits = nullptr, *hist = nullptr, *q_dbg = nullptr;
   float* normed_tmp = nullptr;        // parity reads (GG_READ_EMBED)
+  float* logits_rows = nullptr;       // class-major logits in row order (GG_READ_LOGITS)
   float *rope_local = nullptr, *rope_global = nullptr;   // [ctx][cos|sin][128]
   float* cand_val = nullptr;
   uint32_t *cand_id = nullptr, *top = nullptr, *seen = nullptr;
@@ -1040,6 +1041,7 @@ int gg_finalize(gg_ctx* c) {
   GG_TRY(dalloc(c, &c->normed, (size_t)c->H * 4));
   GG_TRY(dalloc(c, &c->normed_tmp, (size_t)c->H * 4));
   GG_TRY(dalloc(c, &c->logits, (size_t)c->V * 4));
+  GG_TRY(dalloc(c, &c->logits_rows, (size_t)c->V * 4));
   GG_TRY(dalloc(c, &c->hist, (size_t)c->L * c->H * 4));
   GG_TRY(dalloc(c, &c->q_dbg, (size_t)c->L * c->QD * 4));
   GG_TRY(dalloc(c, &c->rope_local, (size_t)c->CTX * kHeadDim * 4));
@@ -1532,15 +1534,12 @@ int gg_read(gg_ctx* c, int32_t what, int32_t layer, void* dst, size_t nbytes) {
   if (nbytes < sz) sz = nbytes;
   GG_TRY(sync(c, "read"));
   if (what == GG_READ_LOGITS && c->logits_cm) {
-    // the persistent kernel's LM head leaves class-major logits:
-    // row c + 256 k at c * (V / 256) + k
-    std::vector<float> cm((size_t)c->V);
-    GG_HIP(c, hipMemcpy(cm.data(), src, (size_t)c->V * 4, hipMemcpyDeviceToHost));
-    const int R = c->V / 256;
-    float* o = (float*)dst;
-    const size_t n = sz / 4;
-    for (size_t r = 0; r < n; ++r) o[r] = cm[(r & 255) * R + (r >> 8)];
-    return GG_OK;
+    // the persistent kernel's LM head leaves class-major logits; put in row
+    // order on the device (the same loop over 262144 strided host floats was
+    // 0.75 of the read's 0.83 ms)
+    GG_TRY(launch_rc(c, launch_logits_rows(c->logits, c->logits_rows, c->V, c->stream), "logits order"));
+    GG_TRY(sync(c, "read"));
+    src = c->logits_rows;
   }
   GG_HIP(c, hipMemcpy(dst, src, sz, hipMemcpyDeviceToHost));
   return GG_OK;
