@@ -228,6 +228,8 @@ struct SelectArgs {
   uint32_t* seen;          // [ceil(V/32)] penalty bitmap
   DevState* st;
   int auto_add;            // add the chosen id to the bitmap
+  int in_use;              // != 0: the sampling parameters are `in`, not DevState's
+  SampleIn in;
   int32_t* host_out;       // optional: mapped pinned host word that also receives the token
 };
 

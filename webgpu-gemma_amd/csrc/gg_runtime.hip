@@ -1675,13 +1675,13 @@ size_t gg_select_workspace_size(int32_t n) {
 // gg_select_logits_noalloc.
 static int select_with_workspace(const float* logits, int32_t n, const uint32_t* seen, const gg_sample* s,
                                  double u, char* ws, void* topk_out, int32_t* out_token, hipStream_t hs) {
-  DevState h{};
-  h.temperature = s->temperature;
-  h.top_p = s->top_p;
-  h.rep_penalty = s->rep_penalty;
-  h.u = u;
-  h.seen_count = seen ? 1 : 0;
   SelectArgs a{};
+  a.in_use = 1;   // the parameters travel as kernel arguments: no upload before the launch
+  a.in.temperature = s->temperature;
+  a.in.top_p = s->top_p;
+  a.in.rep_penalty = s->rep_penalty;
+  a.in.u = u;
+  a.in.seen_count = seen ? 1 : 0;
   a.logits = logits;
   a.V = n;
   a.st = (DevState*)ws;
@@ -1690,12 +1690,10 @@ static int select_with_workspace(const float* logits, int32_t n, const uint32_t*
   a.top = topk_out ? (uint32_t*)topk_out : (uint32_t*)(ws + 256 + (size_t)kSelBlocks * 256 * 8);
   a.seen = seen ? (uint32_t*)seen : (uint32_t*)ws;  // never read when seen_count == 0
   a.auto_add = 0;
-  if (hipMemcpyAsync(ws, &h, sizeof(h), hipMemcpyHostToDevice, hs) != hipSuccess) return GG_ERR_HIP;
   if (launch_select(a, hs)) return GG_ERR_HIP;
-  DevState back{};
-  if (hipMemcpyAsync(&back, ws, sizeof(back), hipMemcpyDeviceToHost, hs) != hipSuccess) return GG_ERR_HIP;
-  if (hipStreamSynchronize(hs) != hipSuccess) return GG_ERR_HIP;
-  *out_token = back.out_token;
+  int32_t token = 0;
+  if (hipMemcpyWithStream(&token, &a.st->out_token, 4, hipMemcpyDeviceToHost, hs) != hipSuccess) return GG_ERR_HIP;
+  *out_token = token;
   return GG_OK;
 }
 
