@@ -142,11 +142,12 @@ struct AttnArgs {
   float* q_dbg;            // decode, optional: normed+roped q of this token
   // batched prefill: prompt row r sits at position pf_start + r; q of every
   // row and k, v of every position that the slice attends to are in operand
-  // order (k_rows_kv); the key tiles of a 32-row query tile are split in
-  // chunks of pf_chunk
+  // order (k_rows_kv); the key tiles of a query tile of 16 pf_rt rows are
+  // split in chunks of pf_chunk
   int pf_start;
   int pf_rows;
   int pf_chunk;
+  int pf_rt;
   const uint16_t* q_frag;
   const uint8_t* kv_planes;
 };
@@ -384,25 +385,34 @@ constexpr int kGemmFewRows = 512;
 inline int gemm_slices(int M) { return M <= kGemmFewRows ? kGemmMaxSlices : 4; }   // O, down
 inline int qkv_slices(int M) { return M <= kGemmFewRows ? kQkvMaxSlices : 2; }
 constexpr int kPrefillChunks = 16;   // key chunks per query tile in the batched prefill attention
-// Most 32-key tiles that a 32-row query tile of a prefill of M rows at `start` reads.
-inline int prefill_max_tiles(int window, int start, int M) {
-  const int full = (start + M + 31) / 32;
-  return window > 0 ? (full < (window + 31 + 31) / 32 + 1 ? full : (window + 31 + 31) / 32 + 1) : full;
+// Most 32-key tiles that a query tile of `rows` rows of a prefill of M rows at `start` reads.
+inline int prefill_max_tiles(int window, int start, int M, int rows) {
+  const int full = (start + M + 31) / 32, local = (window + rows - 1 + 30) / 32 + 1;
+  return window > 0 && local < full ? local : full;
 }
-// Key tiles per chunk: the split (at most kPrefillChunks chunks) with the
-// least modelled time, in tiles of a block on a CU of its own (2 us): rounds
-// of 256 blocks times a chunk's tiles and 2 for its start and end, plus the
-// merge of several chunks (a launch, and the partials written and read).
-inline int prefill_chunk(int window, int start, int M) {
-  const int tiles = prefill_max_tiles(window, start, M), qt = (M + 31) / 32;
-  int best = tiles;
+// Rows per query tile (16 rt) and key tiles per chunk (at most kPrefillChunks
+// chunks): the pair with the least modelled time in us: rounds of 256 blocks
+// times a block's tiles, start and end (both slower with more CUs busy), plus,
+// for several chunks, the merge. 16-row tiles cost more per row but give
+// twice the blocks and halve a block's start, end and partials; they win where
+// 32-row tiles leave CUs idle or need several chunks (64 rows: 7.5 us against
+// 11.7; 2048 rows, window 512: 24 + 7 us for two chunks against 26 + 9 for
+// four of 32-row tiles; 4096 rows: no merge), 32-row tiles on long spans.
+struct PrefillPlan { int rt, chunk; };
+inline PrefillPlan prefill_plan(int window, int start, int M) {
+  PrefillPlan best{2, 1 << 30};
   double best_cost = 0.0;
-  for (int n = 1; n <= kPrefillChunks && n <= tiles; ++n) {
-    const int ct = (tiles + n - 1) / n, nc = (tiles + ct - 1) / ct;
-    const double cost = (double)((qt * nc + 255) / 256) * (ct + 2) + (nc > 1 ? 1.5 + nc * M * 4e-4 : 0.0);
-    if (n == 1 || cost < best_cost) {
-      best_cost = cost;
-      best = ct;
+  for (int rt = 1; rt <= 2; ++rt) {
+    const int tiles = prefill_max_tiles(window, start, M, 16 * rt), qt = (M + 16 * rt - 1) / (16 * rt);
+    for (int n = 1; n <= kPrefillChunks && n <= tiles; ++n) {
+      const int ct = (tiles + n - 1) / n, nc = (tiles + ct - 1) / ct;
+      const double busy = qt * nc < 256 ? qt * nc / 256.0 : 1.0;
+      const double block = rt == 2 ? ct * (2.1 + 0.9 * busy) + 7.0 + 4.0 * busy : ct * (1.25 + 0.6 * busy) + 5.0 + 2.0 * busy;
+      const double cost = ((qt * nc + 255) / 256) * block + (nc > 1 ? 4.3 + nc * M * 6.0e-4 : 0.0);
+      if ((rt == 1 && n == 1) || cost < best_cost) {
+        best_cost = cost;
+        best = {rt, ct};
+      }
     }
   }
   return best;

@@ -872,11 +872,14 @@ __global__ __launch_bounds__(256) void k_select2(SelectArgs a, int nb) {
 //
 // k_rows_kv leaves q, k and v as bf16 hi / lo in MFMA operand order, so the
 // splits are made once per value and staging is a plain copy. Block (x = key
-// chunk, y = query tile) covers 32 prompt rows with four waves, one per query
-// head, on one wave's registers per SIMD: a wave holds its 32 rows' q (128
-// registers) and output (128), so every K and V operand read from LDS feeds
-// two row tiles; 16-row waves, two per SIMD, would read 170 bytes of LDS per
-// MFMA cycle of a CU, above its 128.
+// chunk, y = query tile) covers 16 RT prompt rows (32, or 16 where blocks are
+// few: prefill_plan) with four waves, one per query head, each alone on its
+// SIMD: a wave holds its 32 rows' q (128 registers) and output (128), so every
+// K and V operand read from LDS feeds two row tiles; 16-row waves, two per
+// SIMD, would read 170 bytes of LDS per MFMA cycle of a CU, above its 128.
+// Long spans (32749 ids, 1B shape): matrix cores busy 60% of the cycles at
+// 1.88 GHz, where the kernel that split K and V in every block had 13 to 30%;
+// all attention of that prefill 44.4 -> 28.1 ms.
 //   S^T = K Q^T  on v_mfma_f32_16x16x32_bf16, q scaled by log2(e)/16 before
 //                its split: per 32 dims the products hi.hi, lo.hi and hi.lo,
 //                fp32 accumulate (the dropped lo.lo term is below 2^-16
@@ -940,7 +943,6 @@ __device__ __forceinline__ float pf_xor32_max(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-constexpr int kPfRows = 32;   // query rows per block: two 16-row MFMA tiles
 __device__ __forceinline__ bf16x8 lds_bf16x8(const uint8_t* p) {
   return __builtin_bit_cast(bf16x8, *(const u32x4*)p);
 }
@@ -953,17 +955,20 @@ __device__ __forceinline__ int pf_key_lo(const AttnArgs& a, int pos) {
   return a.window > 0 ? max(0, pos - a.window + 1) : 0;
 }
 
-// Key tiles [*t0, *t1] of query tile qt (kPfRows rows), in *nkc chunks of
+// Key tiles [*t0, *t1] of query tile qt (16 pf_rt rows), in *nkc chunks of
 // pf_chunk tiles.
 __device__ __forceinline__ void pf_tile_span(const AttnArgs& a, int qt, int* t0, int* t1, int* nkc) {
-  const int p_first = a.pf_start + qt * kPfRows;
-  const int p_last = a.pf_start + min(qt * kPfRows + kPfRows - 1, a.pf_rows - 1);
+  const int rows = 16 * a.pf_rt;
+  const int p_first = a.pf_start + qt * rows;
+  const int p_last = a.pf_start + min(qt * rows + rows - 1, a.pf_rows - 1);
   *t0 = pf_key_lo(a, p_first) / kPfKeys;
   *t1 = p_last / kPfKeys;
   *nkc = (*t1 - *t0 + a.pf_chunk) / a.pf_chunk;
 }
 
+template <int RT>
 __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
+  constexpr int kPfRows = 16 * RT;
   __shared__ __align__(16) uint8_t Ks[2][kPfTile];
   __shared__ __align__(16) uint8_t Vs[2][kPfTile];
   const int tid = threadIdx.x, lane = tid & 63, h = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -995,28 +1000,28 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
   copy(tb, 1, Vs[0]);
   copy(min(tb + 1, te - 1), 0, Ks[1]);
 
-  // q of row tiles 2 qt + rt: [tile][head][t][plane][lane][8]; waves past the
+  // q of row tiles RT qt + rt: [tile][head][t][plane][lane][8]; waves past the
   // last head repeat it and write nothing
-  bf16x8 qh[2][8], ql[2][8];
-  const u32x4* qp = (const u32x4*)(a.q_frag + (size_t)(2 * qt * nq + min(h, nq - 1)) * 16 * kHeadDim * 2) + lane;
+  bf16x8 qh[RT][8], ql[RT][8];
+  const u32x4* qp = (const u32x4*)(a.q_frag + (size_t)(RT * qt * nq + min(h, nq - 1)) * 16 * kHeadDim * 2) + lane;
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       qh[rt][t] = __builtin_bit_cast(bf16x8, qp[(size_t)rt * nq * 1024 + t * 128]);
       ql[rt][t] = __builtin_bit_cast(bf16x8, qp[(size_t)rt * nq * 1024 + t * 128 + 64]);
     }
 
-  int prow[2], plo[2];      // this lane's rows: position, first key
-  bool row_ok[2];
+  int prow[RT], plo[RT];      // this lane's rows: position, first key
+  bool row_ok[RT];
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     const int row = qt * kPfRows + 16 * rt + c16;
     row_ok[rt] = row < M;
     prow[rt] = a.pf_start + row;
     plo[rt] = pf_key_lo(a, prow[rt]);
   }
-  // every key of the tile is valid for all 32 rows: all rows exist, the last
+  // every key of the tile is valid for all rows: all rows exist, the last
   // key is at most the first row's position, the first key at least the last
   // row's window start
   const int r_first = a.pf_start + qt * kPfRows;
@@ -1026,22 +1031,27 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
     return rows_full && t * kPfKeys + kPfKeys - 1 <= r_first && t * kPfKeys >= lo_last;
   };
 
-  f32x4 o[2][16];
+  f32x4 o[RT][16];
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[rt][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m[2] = {-INFINITY, -INFINITY}, mb[2] = {0.f, 0.f}, l[2] = {0.f, 0.f};
-  f32x4 s[2][2], nx[2][2];  // [row tile][key tile j]: scores of this and of the next tile
-  uint32_t ph[2][4], pl[2][4];
+  float m[RT], mb[RT], l[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    m[rt] = -INFINITY;
+    mb[rt] = l[rt] = 0.f;
+  }
+  f32x4 s[RT][2], nx[RT][2];  // [row tile][key tile j]: scores of this and of the next tile
+  uint32_t ph[RT][4], pl[RT][4];
 
   // The wave runs alone on its SIMD, so its instruction order is the schedule:
   // it is written out and pinned slot by slot (fence), a few VALU instructions
-  // behind each pair of MFMAs, LDS operands read a whole group ahead.
+  // behind each MFMA or pair, LDS operands read a whole group ahead.
   auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
 
-  // d[rt][j] = K Q^T of the K tile at kb: 8 dim blocks of 6 slots of two MFMAs
-  auto scores = [&](const uint8_t* kb, f32x4 (&d)[2][2], auto slot) __attribute__((always_inline)) {
+  // d[rt][j] = K Q^T of the K tile at kb: 8 dim blocks of 6 slots of RT MFMAs
+  auto scores = [&](const uint8_t* kb, f32x4 (&d)[RT][2], auto slot) __attribute__((always_inline)) {
     bf16x8 k[2][4];
     auto read = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
@@ -1057,7 +1067,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
       for (int q = 0; q < 6; ++q) {   // (product, key tile); both row tiles
         const int pr = q >> 1, j = q & 1;
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
           d[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[t & 1][2 * j + (pr == 1)], pr == 2 ? ql[rt][t] : qh[rt][t],
                                                              t == 0 && pr == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[rt][j], 0, 0, 0);
         slot(t * 6 + q);
@@ -1069,6 +1079,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
   // lane's 16 are 2^(s - reference), added to the row's sum and split
   float p0 = 0.f, p1 = 0.f, h0 = 0.f, h1 = 0.f;
   auto probs = [&](int q) __attribute__((always_inline)) {
+    if (q >= 24 * RT) return;
     const int pair = q / 6, rt = pair >> 2, j = (pair >> 1) & 1, r = 2 * (pair & 1);
     switch (q % 6) {
       case 0:
@@ -1098,7 +1109,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
     }
     if (q % 6 < 2) asm volatile("" : "+v"(p0), "+v"(p1));   // or they sink past the MFMAs
   };
-  // O += P V of the V tile at vb: 16 dim tiles of 3 slots of two MFMAs
+  // O += P V of the V tile at vb: 16 dim tiles of 3 slots of RT MFMAs
   auto weighted = [&](const uint8_t* vb, auto slot) __attribute__((always_inline)) {
     bf16x8 v[3][2];
     auto read = [&](int i) __attribute__((always_inline)) {
@@ -1115,7 +1126,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
 #pragma unroll
       for (int pr = 0; pr < 3; ++pr) {
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
+        for (int rt = 0; rt < RT; ++rt) {
           const u32x4 pf = pr == 1 ? u32x4{pl[rt][0], pl[rt][1], pl[rt][2], pl[rt][3]}
                                    : u32x4{ph[rt][0], ph[rt][1], ph[rt][2], ph[rt][3]};
           o[rt][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pf), v[i % 3][pr == 2], o[rt][i],
@@ -1127,10 +1138,10 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
     }
   };
   // causal / window mask of tile t's scores
-  auto mask = [&](int t, f32x4 (&d)[2][2]) __attribute__((always_inline)) {
+  auto mask = [&](int t, f32x4 (&d)[RT][2]) __attribute__((always_inline)) {
     if (tile_full(t)) return;
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -1142,20 +1153,22 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
   };
   // row maxima of the scores d, one of the lane's 16 per slot, then across
   // the four lane groups
-  float mx[2];
-  auto maxima = [&](const f32x4 (&d)[2][2], int q) __attribute__((always_inline)) {
-    const int rt = (q >> 3) & 1;
-    if (q < 16) mx[rt] = (q & 7) == 0 ? d[rt][0][0] : fmaxf(mx[rt], d[rt][(q >> 2) & 1][q & 3]);
-    else if (q < 18) mx[q - 16] = pf_xor16_max(mx[q - 16]);
-    else if (q < 20) mx[q - 18] = pf_xor32_max(mx[q - 18]);
+  float mx[RT];
+  auto maxima = [&](const f32x4 (&d)[RT][2], int q) __attribute__((always_inline)) {
+    const int rt = q >> 3;
+    if (q < 8 * RT) mx[rt] = (q & 7) == 0 ? d[rt][0][0] : fmaxf(mx[rt], d[rt][(q >> 2) & 1][q & 3]);
+    else if (q < 9 * RT) mx[q - 8 * RT] = pf_xor16_max(mx[q - 8 * RT]);
+    else if (q < 10 * RT) mx[q - 9 * RT] = pf_xor32_max(mx[q - 9 * RT]);
   };
   // moves the softmax reference where a row needs it
   auto settle = [&]() __attribute__((always_inline)) {
-    const bool mv0 = mx[0] > m[0] + 8.f, mv1 = mx[1] > m[1] + 8.f;
-    if (__ballot(mv0 || mv1)) {
+    bool mv[RT], any = false;
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        const float mn = (rt ? mv1 : mv0) ? mx[rt] : m[rt];
+    for (int rt = 0; rt < RT; ++rt) any |= mv[rt] = mx[rt] > m[rt] + 8.f;
+    if (__ballot(any)) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const float mn = mv[rt] ? mx[rt] : m[rt];
         const float nb = mn == -INFINITY ? 0.f : mn;   // a row with no key yet keeps p = 0
         const float alpha = __builtin_amdgcn_exp2f(m[rt] - nb);
         m[rt] = mn;
@@ -1178,7 +1191,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
   scores(Ks[0], s, [](int) {});
   mask(tb, s);
 #pragma unroll
-  for (int q = 0; q < 20; ++q) maxima(s, q);
+  for (int q = 0; q < 10 * RT; ++q) maxima(s, q);
   settle();
   for (int t = tb; t + 1 < te; ++t) {
     const int b = (t - tb) & 1;   // stage of V of tile t; K of tile t + 1 is in the other
@@ -1191,18 +1204,18 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
     weighted(Vs[b], [&](int q) { maxima(nx, q); });
     settle();
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int j = 0; j < 2; ++j) s[rt][j] = nx[rt][j];
     arrived();
     __syncthreads();
   }
 #pragma unroll
-  for (int q = 0; q < 48; ++q) probs(q);
+  for (int q = 0; q < 24 * RT; ++q) probs(q);
   weighted(Vs[(te - 1 - tb) & 1], [](int) {});
   if (h >= nq) return;
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     float lt = l[rt];
     lt += __shfl_xor(lt, 16, 64);
     lt += __shfl_xor(lt, 32, 64);
@@ -1245,7 +1258,7 @@ __global__ __launch_bounds__(256) void k_attn_pf_merge(AttnArgs a) {
   // order, as one thread per dim
   const int row = blockIdx.x, tid = threadIdx.x, nq = a.n_q, h = tid >> 6, d4 = tid & 63;
   int t0, t1, nkc;
-  pf_tile_span(a, row / kPfRows, &t0, &t1, &nkc);
+  pf_tile_span(a, row / (16 * a.pf_rt), &t0, &t1, &nkc);
   if (nkc == 1 || h >= nq) return;
   const float* pr = a.part + (size_t)row * kPrefillChunks * nq * (2 + kHeadDim);
   // chunks in groups of four, each group's loads issued together (clamped
@@ -2132,11 +2145,13 @@ int launch_attention_merge(const AttnArgs& a, int chunks, void* stream) {
 
 int launch_prefill_attention(const AttnArgs& a, int M, void* stream) {
   if (a.n_q < 1 || a.n_q > kAttnMaxQ || M < 1 || a.pf_rows != M || a.pf_start < 0 || a.window < 0 || a.pf_chunk < 1 ||
-      !a.q_frag || !a.kv_planes)
+      (a.pf_rt != 1 && a.pf_rt != 2) || !a.q_frag || !a.kv_planes)
     return (int)hipErrorInvalidValue;
-  const int nkc = (prefill_max_tiles(a.window, a.pf_start, M) + a.pf_chunk - 1) / a.pf_chunk;
+  const int nkc = (prefill_max_tiles(a.window, a.pf_start, M, 16 * a.pf_rt) + a.pf_chunk - 1) / a.pf_chunk;
   if (nkc > kPrefillChunks) return (int)hipErrorInvalidValue;   // `part` holds kPrefillChunks per row
-  hipLaunchKernelGGL(k_attn_pf, dim3(nkc, (M + kPfRows - 1) / kPfRows), dim3(256), 0, (hipStream_t)stream, a);
+  const dim3 grid(nkc, (M + 16 * a.pf_rt - 1) / (16 * a.pf_rt));
+  if (a.pf_rt == 1) hipLaunchKernelGGL(k_attn_pf<1>, grid, dim3(256), 0, (hipStream_t)stream, a);
+  else hipLaunchKernelGGL(k_attn_pf<2>, grid, dim3(256), 0, (hipStream_t)stream, a);
   if (nkc > 1) hipLaunchKernelGGL(k_attn_pf_merge, dim3(M), dim3(256), 0, (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }

@@ -741,7 +741,9 @@ int prefill_slice(gg_ctx* c, const int32_t* d_tokens, int M, int start) {
     at.pf_out = c->pf_attn;
     at.pf_start = start;
     at.pf_rows = M;
-    at.pf_chunk = prefill_chunk(at.window, start, M);
+    const PrefillPlan pp = prefill_plan(at.window, start, M);
+    at.pf_rt = pp.rt;
+    at.pf_chunk = pp.chunk;
     GG_TRY(launch_rc(c, launch_prefill_attention(at, M, s), "prefill attention"));
     const GemmArgs go = gemm_base(c->pf_attn, Ly.o_b, Ly.o_d, c->H, c->QD, M, c->pf_o, nullptr, gemm_slices(M));
     GG_TRY(launch_rc(c, launch_gemm(EPI_OUT, go, s), "prefill o"));
