@@ -364,19 +364,24 @@ int launch_gemm(int epi, const GemmArgs& a, void* stream);
 int launch_rows_embed(const RowArgs& a, void* stream);
 int launch_rows_resid(const RowArgs& a, void* stream);
 int launch_rows_kv(const RowArgs& a, void* stream);
-// Block tiles of the prefill GEMM (rows x features).
-enum GemmTileId { GT_32x64, GT_32x128, GT_32x192, GT_64x128, GT_64x192, GT_64x256, GT_128x256, GT_COUNT };
-struct GemmTile {
-  int mi, nj;       // 16 mi rows, 64 nj features
-  bool out, geglu;  // epilogues it is built for
-  float lat, thr;   // us per 32-wide step: alone on a CU / added by each further block of the CU
+// Block tiles of the prefill GEMM (rows x features, K groups).
+enum GemmTileId {
+  GT_32x64, GT_32x64_K2, GT_32x128, GT_32x128_K2, GT_32x192, GT_64x128, GT_64x128_K2, GT_64x192, GT_64x256,
+  GT_128x256, GT_COUNT
 };
-// lat and thr: least-squares fit of 2000 timings, 16 to 4096 rows x the GEMM
-// shapes of Gemma-3 270M and 1B x 1 to 8 K slices, weights from HBM (12% rms).
+struct GemmTile {
+  int mi, nj, kg;        // 16 mi rows, 64 nj features, kg groups of waves along K
+  // us per 32-wide step of a group, for the C output and for GeGLU (0: not
+  // built): alone on a CU / added by each further block of the CU
+  float lat, thr, glat, gthr;
+};
+// Least-squares fits of 3500 timings, 16 to 4096 rows x the GEMM shapes of
+// Gemma-3 270M and 1B x 1 to 8 K slices, weights from HBM (9 to 17% rms).
 constexpr GemmTile kGemmTiles[GT_COUNT] = {
-    {2, 1, true, false, .182f, .116f}, {2, 2, true, true, .252f, .201f},  {2, 3, true, false, .329f, .297f},
-    {4, 2, true, true, .361f, .355f},  {4, 3, true, false, .463f, .473f}, {4, 4, false, true, .605f, .485f},
-    {8, 4, false, true, .955f, .919f}};
+    {2, 1, 1, .182f, .116f, 0.f, 0.f},     {2, 1, 2, .248f, .298f, 0.f, 0.f},  {2, 2, 1, .252f, .201f, .285f, .175f},
+    {2, 2, 2, .383f, .562f, .430f, .446f}, {2, 3, 1, .329f, .297f, 0.f, 0.f},  {4, 2, 1, .361f, .355f, .386f, .281f},
+    {4, 2, 2, .561f, 1.186f, 0.f, 0.f},    {4, 3, 1, .463f, .473f, 0.f, 0.f},  {4, 4, 1, 0.f, 0.f, .749f, .430f},
+    {8, 4, 1, 0.f, 0.f, 1.133f, .750f}};
 constexpr int kGemmMaxSlices = 8;   // K slices of a prefill GEMM (summed by the consumer)
 constexpr int kQkvMaxSlices = 4;    // ... of the QKV GEMM (summed by k_rows_kv)
 // Slices that the output buffers of an M-row GEMM hold: few rows need more

@@ -1355,16 +1355,23 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, size_t
 // down weights carry their inputs in this order.
 __device__ __forceinline__ int act_slot(int f) { return 2 * (f & 15) + (f >> 4); }
 
-template <int EPI, int MI, int NJ, int PW, int PA, int OCC>
-__global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
+// KG > 1: KG groups of four waves split the block's K steps (its own A stages
+// each) and add their tiles through LDS at the end, in a fixed order: the
+// chain of steps, which bounds a hundred rows, is KG times shorter without
+// more K slices for the consumer, and GeGLU tiles can be split too.
+template <int EPI, int MI, int NJ, int PW, int PA, int OCC, int KG>
+__global__ __launch_bounds__(256 * KG, OCC) void k_gemm(GemmArgs a) {
   static_assert(EPI == EPI_OUT || NJ % 2 == 0, "GeGLU pairs adjacent column tiles");
+  static_assert(KG == 1 || NJ <= 2, "half the groups' tiles fit the A stages");
   constexpr int BM = 16 * MI, BN = 64 * NJ;
   constexpr int AC = (BM * 8 + 255) / 256;   // 16-byte A chunks per thread and step
   constexpr int SL = PW + 1;                 // weight register stages
   static_assert(BM * 8 % 256 == 0, "whole chunks");
-  __shared__ __align__(16) uint8_t As[2][BM * 128];
-  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  __shared__ __align__(16) uint8_t stages[KG][2][BM * 128];
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
+  auto& As = stages[kg];
   const int M = a.M, N = a.N, KB = a.K / 32;
   // Tile order: workgroups go to the XCDs round-robin (from an XCD that
   // depends on earlier dispatches), so the blocks with one value of b % 8
@@ -1380,7 +1387,10 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
   const int kz = L / (NT * MT), Lp = L % (NT * MT);
   const int fm = (Lp / (GROUP * NT)) * GROUP, gm = min(MT - fm, GROUP);
   const int m0 = (fm + (Lp % (GROUP * NT)) % gm) * BM, n0 = ((Lp % (GROUP * NT)) / gm) * BN;
-  const int ns = KB / a.ks, kb0 = kz * ns;   // this block's K slice: 32-blocks [kb0, kb0 + ns)
+  // this block's K slice has KB / ks 32-blocks; a group's are [kb0, kb0 + ns)
+  // of them, and every group goes through the same ng steps (and barriers)
+  const int nb = KB / a.ks, ng = (nb + KG - 1) / KG;
+  const int kb0 = kz * nb + min(kg * ng, nb - 1), ns = KG > 1 ? max(min(ng, nb - kg * ng), 0) : nb;
   const int rows = min(BM, M - m0);
   const uint32_t arow = (uint32_t)KB * 128;
   const int t0 = n0 / 16 + wv * NJ;          // this wave's first 16-row weight tile
@@ -1399,7 +1409,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
   float d[SL][NJ];
   // loads past the slice's end repeat its last step (never used)
   auto load_a = [&](int sl, int s) __attribute__((always_inline)) {
-    const uint32_t so = (uint32_t)(kb0 + min(s, ns - 1)) * 128u;
+    const uint32_t so = (uint32_t)(kb0 + max(min(s, ns - 1), 0)) * 128u;
 #pragma unroll
     for (int i = 0; i < AC; ++i) ar[sl][i] = buf_load16(ra, ga[i], so);
   };
@@ -1408,7 +1418,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
     for (int i = 0; i < AC; ++i) *(u32x4*)&As[st][la[i]] = ar[sl][i];
   };
   auto load_w = [&](int sl, int s) __attribute__((always_inline)) {
-    const int k = kb0 + min(s, ns - 1);
+    const int k = kb0 + max(min(s, ns - 1), 0);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) w[sl][j] = buf_load16(rw, lane * 16, (uint32_t)(j * KB + k) * 1024u);
 #pragma unroll
@@ -1436,6 +1446,10 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
     store_a((u + 1) % PA, st ^ 1);
     load_w((sl + PW) % SL, s + PW);
     load_a((u + 1) % PA, s + 1 + PA);
+    if (KG > 1 && s >= ns) {   // a shorter group only keeps the barriers
+      __syncthreads();
+      return;
+    }
     // the MFMA phase runs at raised wave priority: of the waves on a SIMD the
     // computing one issues ahead of the staging ones
     __builtin_amdgcn_s_setprio(1);
@@ -1481,13 +1495,31 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(GemmArgs a) {
   };
   constexpr int U = SL % 2 == 0 ? SL : 2 * SL;
   static_assert(U % PA == 0, "the A registers rotate with the unroll");
-  for (int s = 0; s < ns; s += U) {
+  for (int s = 0; s < ng; s += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (u > 0 && s + u >= ns) break;
+      if (u > 0 && s + u >= ng) break;
       step(s + u, u);
     }
   }
+  // groups h, 3 h, ... hand their tiles to groups 0, 2 h, ...
+#pragma unroll
+  for (int h = 1; h < KG; h *= 2) {
+    f32x4* x = (f32x4*)&stages[0][0][0] + (size_t)(kg / (2 * h)) * 4 * MI * NJ * 64 + wv * MI * NJ * 64 + lane;
+    if (kg % (2 * h) == h)
+#pragma unroll
+      for (int t = 0; t < MI * NJ; ++t) x[64 * t] = acc[t / NJ][t % NJ];
+    __syncthreads();
+    if (kg % (2 * h) == 0)
+#pragma unroll
+      for (int t = 0; t < MI * NJ; ++t) {
+        const f32x4 y = x[64 * t];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[t / NJ][t % NJ][r] += y[r];
+      }
+    if (2 * h < KG) __syncthreads();
+  }
+  if (kg) return;
 
   // D of a 16x16 tile: lane l, register r -> row 4 (l / 16) + r, col l % 16
   if (EPI == EPI_OUT) {
@@ -2241,17 +2273,17 @@ int launch_dequant(const uint8_t* src, float* out, long long n, void* stream) {
   return (int)hipGetLastError();
 }
 
-template <int EPI, int MI, int NJ, int PW, int PA, int OCC>
+template <int EPI, int MI, int NJ, int PW, int PA, int OCC, int KG = 1>
 static int launch_gemm_t(const GemmArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_gemm<EPI, MI, NJ, PW, PA, OCC>), dim3(a.N / (64 * NJ), (a.M + 16 * MI - 1) / (16 * MI), a.ks),
-                     dim3(256), 0, s, a);
+  hipLaunchKernelGGL((k_gemm<EPI, MI, NJ, PW, PA, OCC, KG>),
+                     dim3(a.N / (64 * NJ), (a.M + 16 * MI - 1) / (16 * MI), a.ks), dim3(256 * KG), 0, s, a);
   return (int)hipGetLastError();
 }
 
 int launch_gemm(int epi, const GemmArgs& a, void* stream) {
   if (a.tile < 0 || a.tile >= GT_COUNT) return (int)hipErrorInvalidValue;
   const GemmTile& t = kGemmTiles[a.tile];
-  if (a.M < 1 || a.N < 64 || a.N % (64 * t.nj) || !(epi == EPI_OUT ? t.out : t.geglu) || a.K < 64 || a.ks < 1 ||
+  if (a.M < 1 || a.N < 64 || a.N % (64 * t.nj) || !((epi == EPI_OUT ? t.lat : t.glat) > 0.f) || a.K < 64 || a.ks < 1 ||
       a.ks > kGemmMaxSlices || a.K % (32 * a.ks) || !a.A || !a.W || !a.D ||
       (epi == EPI_OUT ? !a.C : (!a.act || a.ks != 1)))
     return (int)hipErrorInvalidValue;
@@ -2259,6 +2291,7 @@ int launch_gemm(int epi, const GemmArgs& a, void* stream) {
   if (epi == EPI_GEGLU) {
     switch (a.tile) {
       case GT_32x128: return launch_gemm_t<EPI_GEGLU, 2, 2, 3, 2, 4>(a, s);
+      case GT_32x128_K2: return launch_gemm_t<EPI_GEGLU, 2, 2, 3, 2, 4, 2>(a, s);
       case GT_64x128: return launch_gemm_t<EPI_GEGLU, 4, 2, 3, 2, 3>(a, s);
       case GT_64x256: return launch_gemm_t<EPI_GEGLU, 4, 4, 1, 1, 3>(a, s);
       case GT_128x256: return launch_gemm_t<EPI_GEGLU, 8, 4, 1, 1, 2>(a, s);
@@ -2266,9 +2299,12 @@ int launch_gemm(int epi, const GemmArgs& a, void* stream) {
   } else {
     switch (a.tile) {
       case GT_32x64: return launch_gemm_t<EPI_OUT, 2, 1, 3, 2, 4>(a, s);
+      case GT_32x64_K2: return launch_gemm_t<EPI_OUT, 2, 1, 3, 2, 4, 2>(a, s);
       case GT_32x128: return launch_gemm_t<EPI_OUT, 2, 2, 3, 2, 4>(a, s);
+      case GT_32x128_K2: return launch_gemm_t<EPI_OUT, 2, 2, 3, 2, 4, 2>(a, s);
       case GT_32x192: return launch_gemm_t<EPI_OUT, 2, 3, 3, 2, 3>(a, s);
       case GT_64x128: return launch_gemm_t<EPI_OUT, 4, 2, 3, 2, 3>(a, s);
+      case GT_64x128_K2: return launch_gemm_t<EPI_OUT, 4, 2, 3, 2, 3, 2>(a, s);
       case GT_64x192: return launch_gemm_t<EPI_OUT, 4, 3, 2, 1, 3>(a, s);
     }
   }

@@ -643,27 +643,31 @@ int sync(gg_ctx* c, const char* what) {
 
 
 // Block tile and K slices (up to max_ks, dividing K into whole 32-blocks)
-// that minimise the modelled time: the 32-wide steps of a block times the
-// fitted time of a step with as many blocks on the CU as this launch puts
-// there (kGemmTiles; 0.3 of the round-up to whole blocks per CU counts, the
-// rest overlaps), plus 6 bytes per output of each slice at 5 TB/s for writing
-// it and for the consumer's read (down at 2048 rows: 81 us and 11.5 us in the
-// row kernel with two slices, 70 and 14 us with four). Over the timings that the fit used, the
-// choice is 4% slower than the best tile and split on average and 21% at
-// worst, while the best fixed tile of a matrix is off by 2x at the ends.
+// that minimise the modelled time: the 32-wide steps of a block's longest
+// group times the fitted time of a step with as many blocks on the CU as this
+// launch puts there (kGemmTiles; of the round-up to whole blocks per CU 0.3
+// counts for the C output, whose blocks are many and overlap, 0.8 for GeGLU),
+// 0.3 us for the exchange between groups, plus 6 bytes per output of each
+// slice at 5 TB/s for writing it and for the consumer's read (down at 2048
+// rows: 81 us and 11.5 us in the row kernel with two slices, 70 and 14 us with
+// four). Over the timings that the fits used, the choice is 4.9% (C) and 0.5%
+// (GeGLU) slower than the best tile and split on average, while the best fixed
+// tile of a matrix is off by 2x at the ends.
 void gemm_plan(GemmArgs& g, int max_ks, bool out) {
   const int steps = g.K / 32;
+  const double whole = out ? 0.3 : 0.8;
   double best = 0.0;
   g.tile = -1;
   for (int t = 0; t < GT_COUNT; ++t) {
     const GemmTile& T = kGemmTiles[t];
-    if (g.N % (64 * T.nj) || !(out ? T.out : T.geglu)) continue;
+    const double lat = out ? T.lat : T.glat, thr = out ? T.thr : T.gthr;
+    if (g.N % (64 * T.nj) || !(lat > 0.0)) continue;
     const int tiles = (g.N / (64 * T.nj)) * cdiv(g.M, 16 * T.mi);
     for (int ks = 1; ks <= max_ks; ++ks) {
       if (steps % ks) continue;
       const double blocks = (double)tiles * ks;
-      const double per_cu = 0.7 * std::max(1.0, blocks / 256) + 0.3 * std::ceil(blocks / 256);
-      const double cost = (steps / ks) * (T.lat + T.thr * (per_cu - 1.0)) +
+      const double per_cu = (1.0 - whole) * std::max(1.0, blocks / 256) + whole * std::ceil(blocks / 256);
+      const double cost = cdiv(steps / ks, T.kg) * (lat + thr * (per_cu - 1.0)) + (T.kg > 1 ? 0.3 : 0.0) +
                           (out ? ks * ((double)g.M * g.N * 6 / 5e6) : 0.0);
       if (g.tile < 0 || cost < best) {
         best = cost;
