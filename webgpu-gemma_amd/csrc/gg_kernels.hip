@@ -2294,7 +2294,7 @@ int launch_gemm(int epi, const GemmArgs& a, void* stream) {
       case GT_32x128_K2: return launch_gemm_t<EPI_GEGLU, 2, 2, 3, 2, 4, 2>(a, s);
       case GT_64x128: return launch_gemm_t<EPI_GEGLU, 4, 2, 3, 2, 3>(a, s);
       case GT_64x256: return launch_gemm_t<EPI_GEGLU, 4, 4, 1, 1, 3>(a, s);
-      case GT_128x256: return launch_gemm_t<EPI_GEGLU, 8, 4, 1, 1, 2>(a, s);
+      case GT_128x256: return launch_gemm_t<EPI_GEGLU, 8, 4, 2, 1, 2>(a, s);
     }
   } else {
     switch (a.tile) {
