@@ -1333,9 +1333,9 @@ __global__ __launch_bounds__(256) void k_attn_pf_merge(AttnArgs a) {
 // load, a 128 x 256 one 63% at 1.83 GHz, in the same time), at a hundred rows
 // the latency of a step. The larger tiles use each weight for more rows and
 // win where weights come from HBM, the small ones start more blocks. Gate/up
-// of the 1B shape (N 13824, K 1152), weights cold: 4096 rows 283 -> 230 us,
-// 2048 rows 155 -> 125 us, 187 rows 33 -> 27 us against a 128 x 128 tile with
-// both operands in LDS; gate/up of the 270M shape at 64 rows 20 -> 8.5 us.
+// of the 1B shape (N 13824, K 1152), weights cold: 4096 rows 283 -> 229 us,
+// 2048 rows 155 -> 129 us, 187 rows 33 -> 27 us against a 128 x 128 tile with
+// both operands in LDS; gate/up of the 270M shape at 64 rows 20 -> 8.8 us.
 //
 // A rows are [K / 32][hi 32 | lo 32] bf16: one 128-byte line per 32-block.
 // In LDS a 16-row tile's (plane, 8-wide chunk g) is 256 bytes of 16 rows, row
