@@ -36,6 +36,7 @@
 
 #include "gg_device.h"
 #include "gg_internal.h"
+#include "gg_pf_schedule.h"
 
 namespace gg {
 
@@ -891,7 +892,8 @@ __global__ __launch_bounds__(256) void k_select2(SelectArgs a, int nb) {
 //                (keys 8 g .. 8 g + 7 in order), B = V^T per dim; tile 2 k +
 //                e column c is dim 32 k + 2 c + e, so lane l holds O[row
 //                4 g + r] of adjacent dims and stores them as one word.
-// Pipeline of 32-key tiles, one barrier each: while tile t's exponentials and
+// Pipeline of 32-key tiles, one barrier each (pf_schedule_run, and one more
+// behind the first tile's scores): while tile t's exponentials and
 // splits run in the issue slots between the MFMAs of tile t + 1's scores and
 // its P V follows, the next K and V tiles go to the other LDS stage by DMA
 // (64 KB per tile, two stages, no registers).
@@ -983,8 +985,9 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
   // M0 + offset; the offset counts on both sides). Inline asm, because the
   // compiler would wait for every DMA in flight before any LDS read; arrived()
   // waits for them explicitly before the barrier that precedes their readers.
-  auto copy = [&](int t, int part, uint8_t* lds) __attribute__((always_inline)) {
+  auto stage = [&](int t, int part, int st) __attribute__((always_inline)) {
     const uint8_t* src = a.kv_planes + (size_t)t * kKvTileBytes + part * kPfTile + h * 8192;
+    uint8_t* lds = part ? Vs[st] : Ks[st];
     const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + h * 8192;
 #pragma unroll
     for (int half = 0; half < 2; ++half)
@@ -996,9 +999,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
           : "memory", "m0");
   };
   auto arrived = []() __attribute__((always_inline)) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-  copy(tb, 0, Ks[0]);
-  copy(tb, 1, Vs[0]);
-  copy(min(tb + 1, te - 1), 0, Ks[1]);
+  pf_schedule_fill(tb, te, stage);
 
   // q of row tiles RT qt + rt: [tile][head][t][plane][lane][8]; waves past the
   // last head repeat it and write nothing
@@ -1186,33 +1187,30 @@ __global__ __launch_bounds__(256, 1) void k_attn_pf(AttnArgs a) {
     }
   };
 
-  arrived();
-  __syncthreads();
-  scores(Ks[0], s, [](int) {});
-  mask(tb, s);
+  auto barrier = []() __attribute__((always_inline)) { __syncthreads(); };
+  auto first = [&](int t, int ks) __attribute__((always_inline)) {
+    scores(Ks[ks], s, [](int) {});
+    mask(t, s);
 #pragma unroll
-  for (int q = 0; q < 10 * RT; ++q) maxima(s, q);
-  settle();
-  for (int t = tb; t + 1 < te; ++t) {
-    const int b = (t - tb) & 1;   // stage of V of tile t; K of tile t + 1 is in the other
-    // V stage b ^ 1 (tile t - 1) and K stage b (tile t) were last read before
-    // the previous barrier
-    copy(t + 1, 1, Vs[b ^ 1]);
-    copy(min(t + 2, te - 1), 0, Ks[b]);
-    scores(Ks[b ^ 1], nx, probs);
+    for (int q = 0; q < 10 * RT; ++q) maxima(s, q);
+    settle();
+  };
+  auto step = [&](int t, int ks, int vs) __attribute__((always_inline)) {
+    scores(Ks[ks], nx, probs);
     mask(t + 1, nx);
-    weighted(Vs[b], [&](int q) { maxima(nx, q); });
+    weighted(Vs[vs], [&](int q) { maxima(nx, q); });
     settle();
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int j = 0; j < 2; ++j) s[rt][j] = nx[rt][j];
-    arrived();
-    __syncthreads();
-  }
+  };
+  auto last = [&](int, int vs) __attribute__((always_inline)) {
 #pragma unroll
-  for (int q = 0; q < 24 * RT; ++q) probs(q);
-  weighted(Vs[(te - 1 - tb) & 1], [](int) {});
+    for (int q = 0; q < 24 * RT; ++q) probs(q);
+    weighted(Vs[vs], [](int) {});
+  };
+  pf_schedule_run(tb, te, stage, arrived, barrier, first, step, last);
   if (h >= nq) return;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
