@@ -252,7 +252,10 @@ int gg_q8_0_dequant(const void* src_gguf, float* out, int64_t n_elems, void* str
 /* Token selection over a device logits vector (argmax / topk256 / sampler,
  * shaders.ts:327-384 + engine.ts:862-901). seen_bitmap: ceil(n/32) u32 words
  * (may be NULL when rep_penalty <= 1). topk_out: 256 x {f32, u32} or NULL.
- * Workspace: gg_select_workspace_size() bytes. out_token: host pointer. */
+ * Workspace: gg_select_workspace_size() bytes. out_token: host pointer.
+ * Waits for the stream and returns once the selection is done, so a stream
+ * under HIP graph capture is refused with GG_ERR_HIP (nothing is recorded,
+ * the capture stays valid). */
 size_t gg_select_workspace_size(int32_t n);
 int gg_select_logits(const float* logits, int32_t n, const uint32_t* seen_bitmap,
                      const gg_sample* s, double u, void* workspace, void* topk_out,
@@ -260,12 +263,11 @@ int gg_select_logits(const float* logits, int32_t n, const uint32_t* seen_bitmap
 
 /* gg_select_logits without a workspace argument and without any device
  * allocation: for callers that cannot allocate (tight serving loops,
- * harnesses that forbid hipMalloc). No counterpart in the reference. It is
- * not usable under HIP graph capture: it copies the sampling state from host
- * memory and synchronizes the stream, and returns only once the selection
- * has finished. The workspace is a static 67,840-byte device array, one
- * copy per GPU, held until the process ends; its address is looked up once
- * per device on the first call there. Every call on one GPU shares that
+ * harnesses that forbid hipMalloc). No counterpart in the reference. It
+ * waits for the stream and refuses capture as gg_select_logits does. The
+ * workspace is a static 67,840-byte device array, one copy per GPU, held
+ * until the process ends; its address is looked up once per device on the
+ * first call there. Every call on one GPU shares that
  * array: calls that overlap on one GPU (other streams or host threads) race.
  * Returns GG_ERR_INVALID, with a message on stderr, when n would need a
  * larger workspace than the static one (gg_select_workspace_size(n) bytes;

@@ -1681,6 +1681,10 @@ size_t gg_select_workspace_size(int32_t n) {
 // gg_select_logits_noalloc.
 static int select_with_workspace(const float* logits, int32_t n, const uint32_t* seen, const gg_sample* s,
                                  double u, char* ws, void* topk_out, int32_t* out_token, hipStream_t hs) {
+  // a capturing stream is refused before anything is recorded: the copy of the
+  // id below cannot be captured and would end the caller's capture
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(hs, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return GG_ERR_HIP;
   SelectArgs a{};
   a.in_use = 1;   // the parameters travel as kernel arguments: no upload before the launch
   a.in.temperature = s->temperature;
