@@ -1960,6 +1960,12 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t* __restrict__ src
 // (4352 bytes, a multiple of 16) through LDS in 16-byte loads and writes 4096
 // floats in 16-byte stores; the byte loads and 4-byte stores above keep a
 // quarter of the bytes in flight (8 M values, 40 MB: 12.4 -> 7.9 us).
+// One block's chain (load, LDS, barrier, store) is longer than the byte
+// kernel's, so dequant_wide takes it where the byte kernel has well more blocks
+// than the chip holds at once (8 per CU: 524288 values), or for up to three
+// blocks. Kernel times back to back, wide against byte: 128 values 1.50 / 1.32 us, 4096 1.71 / 1.97, 12288 1.98 / 1.98,
+// 65536 2.60 / 2.00, 524288 2.81 / 2.45, 786432 2.94 / 2.93, 1 M 3.07 / 3.22,
+// 2 M 3.84 / 4.68.
 constexpr int kDeqBlocks = 128;
 __global__ __launch_bounds__(256) void k_dequant16(const uint8_t* __restrict__ src, float* __restrict__ out,
                                                    long long nblk) {
@@ -2258,9 +2264,12 @@ int launch_logits_rows(const float* cm, float* out, int V, void* stream) {
   return (int)hipGetLastError();
 }
 
+// Sizes for k_dequant16 (measured beside it).
+static bool dequant_wide(long long n) { return n >= 786432 || (n >= 512 && n <= 3 * 32 * kDeqBlocks); }
+
 int launch_dequant(const uint8_t* src, float* out, long long n, void* stream) {
   if (n <= 0) return 0;
-  if (n % 32 == 0 && ((uintptr_t)src | (uintptr_t)out) % 16 == 0) {
+  if (n % 32 == 0 && ((uintptr_t)src | (uintptr_t)out) % 16 == 0 && dequant_wide(n)) {
     const long long nblk = n / 32;
     hipLaunchKernelGGL(k_dequant16, dim3((unsigned)((nblk + kDeqBlocks - 1) / kDeqBlocks)), dim3(256), 0,
                        (hipStream_t)stream, src, out, nblk);
