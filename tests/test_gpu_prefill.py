@@ -105,8 +105,9 @@ def test_1b_batched_prefill_2048_matches_token_by_token(gpu, mode):
 def test_1b_batched_prefill_short_turns_match_token_by_token(gpu):
     """Gemma-3-1B shapes, gemma3 attention: two short turns (300 prompt ids,
     then 77 more at position 300) batched against the token-by-token path.
-    Row counts this small run the QKV, O and down GEMMs on 96-wide tiles
-    (K split in 2 and 4), the 2048-row prefill only its QKV GEMM."""
+    Row counts this small run the QKV, O and down GEMMs on 32- and 64-row
+    tiles with K split over blocks and over groups of waves, the 2048-row
+    prefill mostly on larger tiles."""
     shape = synth.GEMMA3_1B.with_ctx(4096).gemma3_mode()
     say("1b short batched turns, 300 + 77 ids")
     if "1b" not in _MODELS:
@@ -141,7 +142,7 @@ def test_1b_batched_prefill_short_turns_match_token_by_token(gpu):
 def test_1b_batched_prefill_ragged_slices_long_span(gpu):
     """Gemma-3-1B shapes at contextLength 8192, gemma3 attention: a 6000-id
     prompt prefilled in ragged batched slices (2500 + 2500 + 1000 rows: no
-    slice length or start is a multiple of the 128-row GEMM tile, and the
+    slice length or start is a multiple of a GEMM tile of 32 to 128 rows, and the
     global layers' key spans reach 6000) against the token-by-token path;
     then decode steps past 4096 positions (256-chunk attention + merge)."""
     shape = synth.GEMMA3_1B.with_ctx(8192).gemma3_mode()
@@ -224,7 +225,7 @@ def test_1b_batched_prefill_32k_matches_token_path_and_oracle(gpu):
 
 
 def test_270m_batched_prefill_matches_oracle(gpu):
-    """Gemma-3-270M architecture (hidden 640: 128-wide GEMM tiles with a K
+    """Gemma-3-270M architecture (hidden 640: 32-row GEMM tiles with a K
     split, 64-row prompt), gemma3 attention: the 64-id prompt in one batched
     prefill against the oracle's token-by-token prefill (per-layer hidden,
     K/V cache, normed hidden), then 32 greedy tokens identical to it."""

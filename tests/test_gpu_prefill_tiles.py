@@ -16,7 +16,7 @@ _MODELS = {}
 SHAPES = {
     "270m": synth.Shape(hidden=640, layers=2, n_q=4, inter=2048, vocab=4096, ctx=4096),
     "1b": synth.Shape(hidden=1152, layers=2, n_q=4, inter=6912, vocab=4096, ctx=4096),
-    # odd block counts: 10 and 18 32-blocks per row, 2 query heads
+    # few 32-blocks per row (4 and 18), 2 query heads
     "ragged": synth.Shape(hidden=128, layers=2, n_q=2, inter=576, vocab=4096, ctx=4096),
 }
 
