@@ -366,7 +366,7 @@ int launch_rows_resid(const RowArgs& a, void* stream);
 int launch_rows_kv(const RowArgs& a, void* stream);
 // Block tiles of the prefill GEMM (rows x features, K groups).
 enum GemmTileId {
-  GT_32x64, GT_32x64_K2, GT_32x128, GT_32x128_K2, GT_32x192, GT_64x128, GT_64x128_K2, GT_64x192, GT_64x256,
+  GT_32x64, GT_32x64_K2, GT_32x128, GT_32x128_K2, GT_64x128, GT_64x128_K2, GT_64x192, GT_64x256,
   GT_128x256, GT_COUNT
 };
 struct GemmTile {
@@ -379,7 +379,7 @@ struct GemmTile {
 // Gemma-3 270M and 1B x 1 to 8 K slices, weights from HBM (9 to 17% rms).
 constexpr GemmTile kGemmTiles[GT_COUNT] = {
     {2, 1, 1, .182f, .116f, 0.f, 0.f},     {2, 1, 2, .248f, .298f, 0.f, 0.f},  {2, 2, 1, .252f, .201f, .285f, .175f},
-    {2, 2, 2, .383f, .562f, .430f, .446f}, {2, 3, 1, .329f, .297f, 0.f, 0.f},  {4, 2, 1, .361f, .355f, .386f, .281f},
+    {2, 2, 2, .383f, .562f, .430f, .446f}, {4, 2, 1, .361f, .355f, .386f, .281f},
     {4, 2, 2, .561f, 1.186f, 0.f, 0.f},    {4, 3, 1, .463f, .473f, 0.f, 0.f},  {4, 4, 1, 0.f, 0.f, .749f, .430f},
     {8, 4, 1, 0.f, 0.f, 1.133f, .750f}};
 constexpr int kGemmMaxSlices = 8;   // K slices of a prefill GEMM (summed by the consumer)

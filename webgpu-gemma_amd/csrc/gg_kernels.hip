@@ -2309,7 +2309,6 @@ int launch_gemm(int epi, const GemmArgs& a, void* stream) {
       case GT_32x64_K2: return launch_gemm_t<EPI_OUT, 2, 1, 3, 2, 4, 2>(a, s);
       case GT_32x128: return launch_gemm_t<EPI_OUT, 2, 2, 3, 2, 4>(a, s);
       case GT_32x128_K2: return launch_gemm_t<EPI_OUT, 2, 2, 3, 2, 4, 2>(a, s);
-      case GT_32x192: return launch_gemm_t<EPI_OUT, 2, 3, 3, 2, 3>(a, s);
       case GT_64x128: return launch_gemm_t<EPI_OUT, 4, 2, 3, 2, 3>(a, s);
       case GT_64x128_K2: return launch_gemm_t<EPI_OUT, 4, 2, 3, 2, 3, 2>(a, s);
       case GT_64x192: return launch_gemm_t<EPI_OUT, 4, 3, 2, 1, 3>(a, s);
