@@ -72,7 +72,9 @@ typedef struct gg_config {
   int32_t attention_mode;   /* GG_ATTN_* (documentation of intent; window/theta decide) */
   int32_t prefill_batch;    /* 0: gg_prefill runs the decode pass per token like the reference
                                (engine.ts:923-928); > 0: prompt rows per batched MFMA prefill
-                               slice (no reference counterpart) */
+                               slice (no reference counterpart). Adds device memory: a second
+                               copy of the layer weights (2.13 bytes per weight), about 150 KB
+                               per slice row at the 1B shape, 2 KB per context position */
 } gg_config;
 
 /* Sampling options of one selection (GenerateOptions, types.ts:65-78), kept

@@ -173,7 +173,8 @@ struct GemmArgs {
                            // gate / up rows alternate in groups of 16 (16 gate rows, then their up rows)
 };
 
-// Row-wise prefill helpers: one block per prompt row.
+// Row-wise prefill helpers: one block per prompt row, k_rows_kv one per eight
+// aligned positions.
 struct RowArgs {
   int M, H;
   float eps;
@@ -376,7 +377,10 @@ struct GemmTile {
   float lat, thr, glat, gthr;
 };
 // Least-squares fits of 3500 timings, 16 to 4096 rows x the GEMM shapes of
-// Gemma-3 270M and 1B x 1 to 8 K slices, weights from HBM (9 to 17% rms).
+// Gemma-3 270M and 1B x 1 to 8 K slices, weights from HBM (9 to 17% rms; the
+// 128 x 256 line with its weights one step ahead, they are two ahead now).
+// Against traces of whole prefills of the 1B shape: gate/up 118 us modelled,
+// 124 measured at 2048 rows, 22 and 27 at 187; down 87 and 64, 10 and 13.
 constexpr GemmTile kGemmTiles[GT_COUNT] = {
     {2, 1, 1, .182f, .116f, 0.f, 0.f},     {2, 1, 2, .248f, .298f, 0.f, 0.f},  {2, 2, 1, .252f, .201f, .285f, .175f},
     {2, 2, 2, .383f, .562f, .430f, .446f}, {4, 2, 1, .361f, .355f, .386f, .281f},

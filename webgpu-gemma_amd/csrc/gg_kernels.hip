@@ -878,9 +878,10 @@ __global__ __launch_bounds__(256) void k_select2(SelectArgs a, int nb) {
 // SIMD: a wave holds its 32 rows' q (128 registers) and output (128), so every
 // K and V operand read from LDS feeds two row tiles; 16-row waves, two per
 // SIMD, would read 170 bytes of LDS per MFMA cycle of a CU, above its 128.
-// Long spans (32749 ids, 1B shape): matrix cores busy 60% of the cycles at
-// 1.88 GHz, where the kernel that split K and V in every block had 13 to 30%;
-// all attention of that prefill 44.4 -> 28.1 ms.
+// Long spans (global layers of 32760 ids, 1B shape): matrix cores busy 61% of
+// the cycles at 1.85 GHz; 27% in 16-row tiles over a 512 window. All attention
+// of that prefill with its merge takes 29.9 ms, 49.0 with the kernel that split
+// K and V in every block.
 //   S^T = K Q^T  on v_mfma_f32_16x16x32_bf16, q scaled by log2(e)/16 before
 //                its split: per 32 dims the products hi.hi, lo.hi and hi.lo,
 //                fp32 accumulate (the dropped lo.lo term is below 2^-16
@@ -1326,14 +1327,16 @@ __global__ __launch_bounds__(256) void k_attn_pf_merge(AttnArgs a) {
 // in flight in registers). A 64 x 256 block so reads 16 bytes of LDS per
 // MFMA cycle and SIMD where a 2 x 2 wave layout with W in LDS too read 24 and
 // wrote 12, and its operand reads are prefetched one row tile ahead.
-// What bounds it: at thousands of rows the power limit (a 64 x 256 tile keeps
-// the matrix cores busy 71% of the cycles at the 1.64 GHz left under that
-// load, a 128 x 256 one 63% at 1.83 GHz, in the same time), at a hundred rows
-// the latency of a step. The larger tiles use each weight for more rows and
-// win where weights come from HBM, the small ones start more blocks. Gate/up
-// of the 1B shape (N 13824, K 1152), weights cold: 4096 rows 283 -> 229 us,
-// 2048 rows 155 -> 129 us, 187 rows 33 -> 27 us against a 128 x 128 tile with
-// both operands in LDS; gate/up of the 270M shape at 64 rows 20 -> 8.8 us.
+// What bounds it: at thousands of rows the cold weights of every layer and the
+// power limit (in a prefill a 128 x 256 tile keeps the matrix cores busy 54% of
+// the cycles at 1.83 GHz over 2048 rows, 57% at 1.92 over 4096; alone with warm
+// weights 63% at 1.83 GHz, a 64 x 256 one 71% at 1.64, in the same time), at a
+// hundred rows the latency of a step. The larger tiles use each weight for more
+// rows and win where weights come from HBM, the small ones start more blocks.
+// Gate/up of the 1B shape (N 13824, K 1152), weights cold: 4096 rows 283 -> 222
+// to 229 us, 2048 rows 155 -> 124 to 129 us, 187 rows 33 -> 27 us against a
+// 128 x 128 tile with both operands in LDS (ranges: two cards); gate/up of the
+// 270M shape at 64 rows 20 -> 8.5 us.
 //
 // A rows are [K / 32][hi 32 | lo 32] bf16: one 128-byte line per 32-block.
 // In LDS a 16-row tile's (plane, 8-wide chunk g) is 256 bytes of 16 rows, row
@@ -1356,7 +1359,9 @@ __device__ __forceinline__ int act_slot(int f) { return 2 * (f & 15) + (f >> 4);
 // KG > 1: KG groups of four waves split the block's K steps (its own A stages
 // each) and add their tiles through LDS at the end, in a fixed order: the
 // chain of steps, which bounds a hundred rows, is KG times shorter without
-// more K slices for the consumer, and GeGLU tiles can be split too.
+// more K slices for the consumer, and GeGLU tiles can be split too. The plan
+// also takes it at up to a few thousand rows where N is small (64 x 128, N 640,
+// 3264 rows).
 template <int EPI, int MI, int NJ, int PW, int PA, int OCC, int KG>
 __global__ __launch_bounds__(256 * KG, OCC) void k_gemm(GemmArgs a) {
   static_assert(EPI == EPI_OUT || NJ % 2 == 0, "GeGLU pairs adjacent column tiles");
@@ -2301,6 +2306,9 @@ int launch_gemm(int epi, const GemmArgs& a, void* stream) {
       case GT_32x128_K2: return launch_gemm_t<EPI_GEGLU, 2, 2, 3, 2, 4, 2>(a, s);
       case GT_64x128: return launch_gemm_t<EPI_GEGLU, 4, 2, 3, 2, 3>(a, s);
       case GT_64x256: return launch_gemm_t<EPI_GEGLU, 4, 4, 1, 1, 3>(a, s);
+      // two steps of weights in flight spill 9 of its 256 registers (40 bytes a
+      // lane, reloaded once per six steps); one step needs 238 and none, and is
+      // slower where weights come from HBM: 2048 ids 8.01 against 7.87 ms
       case GT_128x256: return launch_gemm_t<EPI_GEGLU, 8, 4, 2, 1, 2>(a, s);
     }
   } else {
